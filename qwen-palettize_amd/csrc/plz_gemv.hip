@@ -637,6 +637,104 @@ __host__ __device__ constexpr int pl_nx(int M) {
   return (pl_chunk(M) + WAVES * 1024 - 1) / (WAVES * 1024);
 }
 typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// The two e4m3 pieces of four finite x (two words of bf16) under the scale 1 / inv, one byte each:
+// x inv = p1 + p2 with p1 = e4m3(x inv) and p2 = e4m3(x inv - p1).
+__device__ __forceinline__ void x_pieces4(uint32_t b01, uint32_t b23, float inv, uint32_t& w1,
+                                          uint32_t& w2) {
+  const float v[4] = {bf2f(b01 & 0xffffu) * inv, bf2f(b01 >> 16) * inv, bf2f(b23 & 0xffffu) * inv,
+                      bf2f(b23 >> 16) * inv};
+  int q1 = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+  q1 = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], q1, true);
+  // the remainders are exact
+  int q2 = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] - __builtin_amdgcn_cvt_f32_fp8(q1, 0),
+                                           v[1] - __builtin_amdgcn_cvt_f32_fp8(q1, 1), 0, false);
+  q2 = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] - __builtin_amdgcn_cvt_f32_fp8(q1, 2),
+                                       v[3] - __builtin_amdgcn_cvt_f32_fp8(q1, 3), q2, true);
+  w1 = (uint32_t)q1;
+  w2 = (uint32_t)q2;
+}
+// NaN and +-inf among the four become e4m3 NaN in both pieces, so their token's outputs go NaN.
+__device__ __forceinline__ void x_nonfinite4(uint32_t b01, uint32_t b23, uint32_t& w1,
+                                             uint32_t& w2) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if ((((i < 2 ? b01 : b23) >> (16 * (i & 1))) & 0x7f80u) == 0x7f80u) {
+      w1 |= 0x7fu << (8 * i);
+      w2 |= 0x7fu << (8 * i);
+    }
+}
+// A row's palette group from its lookup words (bf16 bits: high bytes in hi, low bytes in lo) as
+// the fp32 coefficients of the bit planes: w = p0 + c1 b0 + c2 b1 + c3 b0 b1.
+__device__ __forceinline__ void plane_coefs(uint32_t lo, uint32_t hi, float& p0, float& c1,
+                                            float& c2, float& c3) {
+  p0 = __uint_as_float(perm(hi, lo, 0x04000c0cu));
+  const float p1 = __uint_as_float(perm(hi, lo, 0x05010c0cu));
+  const float p2 = __uint_as_float(perm(hi, lo, 0x06020c0cu));
+  const float p3 = __uint_as_float(perm(hi, lo, 0x07030c0cu));
+  c1 = p1 - p0;
+  c2 = p2 - p0;
+  c3 = (p3 - p2) - c1;
+}
+
+// Lane c of 16: x pieces, scale byte and stage sum of token t, from its 16 values
+// x[k0 .. k0 + 15], k0 = prep_k(c), into the stage's chunk (pl_chunk layout); lanes that are not
+// live take part in the sums only. The adds run in a fixed order.
+__device__ __forceinline__ int prep_k(int c) {
+  return 128 * (c >> 3) + 64 * (c & 1) + 16 * ((c >> 1) & 3);
+}
+__device__ __forceinline__ void prep_token(const uint4 v0, const uint4 v1, bool live, int c, int t,
+                                           int M, uint8_t* ch) {
+  const uint32_t b[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+  // the largest finite exponent (the largest magnitude's, unless a value is not finite) sets the
+  // scale
+  float sum = 0.f;
+  u16x2 mag = {0, 0};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    mag = __builtin_elementwise_max(mag, __builtin_bit_cast(u16x2, b[i] & 0x7fff7fffu));
+    sum += bf2f(b[i] & 0xffffu);
+    sum += bf2f(b[i] >> 16);
+  }
+  int emax = (mag.x > mag.y ? mag.x : mag.y) >> 7;
+  const bool odd = emax == 0xff;  // a NaN or infinity among the lane's values
+  if (odd) {
+    emax = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int e0 = (int)((b[i] >> 7) & 0xffu), e1 = (int)((b[i] >> 23) & 0xffu);
+      emax = e0 != 0xff && e0 > emax ? e0 : emax;
+      emax = e1 != 0xff && e1 > emax ? e1 : emax;
+    }
+  }
+#pragma unroll
+  for (int off = 8; off >= 1; off >>= 1) {  // over the 16 lanes of the token, fixed order
+    const int oe = __shfl_xor(emax, off);
+    emax = oe > emax ? oe : emax;
+    sum += __shfl_xor(sum, off);
+  }
+  if (!live) return;
+  // scale 2^s = 2^(E - 7), E the unbiased exponent of the stage's largest finite |x| plus
+  // one: |x| / 2^s < 256, well inside e4m3's 448; e8 = s + 127
+  const int e8 = emax >= 7 ? emax - 7 : 0;
+  const float inv = __builtin_bit_cast(float, (uint32_t)(254 - e8) << 23);  // 2^-s
+  uint32_t w1[4], w2[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x_pieces4(b[2 * i], b[2 * i + 1], inv, w1[i], w2[i]);
+  if (odd)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x_nonfinite4(b[2 * i], b[2 * i + 1], w1[i], w2[i]);
+  const int m0 = 2 * t, m1 = 2 * t + 1;
+  *reinterpret_cast<uint4*>(ch + m0 * 256 + ((c ^ (m0 & 15)) << 4)) =
+      make_uint4(w1[0], w1[1], w1[2], w1[3]);
+  *reinterpret_cast<uint4*>(ch + m1 * 256 + ((c ^ (m1 & 15)) << 4)) =
+      make_uint4(w2[0], w2[1], w2[2], w2[3]);
+  if (c == 0) {
+    ch[512 * M + t] = (uint8_t)e8;
+    reinterpret_cast<float*>(ch + 512 * M + 16)[t] = sum;
+  }
+}
 
 // One wave per linear, PREP_STAGES stages and PREP_TOKENS tokens: lane 16 g + c makes 16-byte
 // piece c of work item 4 i + g, the items being the (token, stage) pairs of the wave's tokens
@@ -661,63 +759,17 @@ __global__ __launch_bounds__(64) void gemv_pl_prep_kernel(const plz_gemv_desc* _
   if (s0 >= stages || dd.N == 0) return;  // uniform per block
   const int ns = stages - s0 < PREP_STAGES ? stages - s0 : PREP_STAGES;
   const int lane = threadIdx.x, c = lane & 15, g = lane >> 4;
-  const int k0 = 128 * (c >> 3) + 64 * (c & 1) + 16 * ((c >> 1) & 3);
+  const int k0 = prep_k(c);
   for (int w0 = 0; w0 < mt * ns; w0 += 4) {
     const int w = w0 + g, t = t0 + w % mt, s = s0 + w / mt;
     const bool live = w < mt * ns;
-    uint32_t b[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    uint4 v0 = make_uint4(0, 0, 0, 0), v1 = v0;
     if (live) {
       const uint4* src = reinterpret_cast<const uint4*>(dd.x + (int64_t)t * dd.K + (int64_t)s * KC + k0);
-      const uint4 v0 = src[0], v1 = src[1];
-      b[0] = v0.x; b[1] = v0.y; b[2] = v0.z; b[3] = v0.w;
-      b[4] = v1.x; b[5] = v1.y; b[6] = v1.z; b[7] = v1.w;
+      v0 = src[0];
+      v1 = src[1];
     }
-    float v[16];
-    int emax = 0;
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const uint32_t h = (b[i / 2] >> (16 * (i & 1))) & 0xffffu;
-      v[i] = bf2f(h);
-      const int e = (int)((h >> 7) & 0xffu);
-      emax = e != 0xff && e > emax ? e : emax;  // the finite values set the scale
-      sum += v[i];
-    }
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) {  // over the 16 lanes of the item, fixed order
-      const int oe = __shfl_xor(emax, off);
-      emax = oe > emax ? oe : emax;
-      sum += __shfl_xor(sum, off);
-    }
-    if (!live) continue;
-    uint8_t* ch = ws + ((int64_t)d * max_stages + s) * pl_chunk(M);
-    // scale 2^s = 2^(E - 7), E the unbiased exponent of the stage's largest finite |x| plus
-    // one: |x| / 2^s < 256, well inside e4m3's 448; e8 = s + 127
-    const int e8 = emax >= 7 ? emax - 7 : 0;
-    const float inv = __builtin_bit_cast(float, (uint32_t)(254 - e8) << 23);  // 2^-s
-    uint32_t w1[4] = {0, 0, 0, 0}, w2[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float xs = v[i] * inv;
-      uint32_t p1 = 0x7fu, p2 = 0x7fu;  // NaN and +-inf: e4m3 NaN, the token's outputs go NaN
-      if (__builtin_isfinite(xs)) {
-        const int q1 = __builtin_amdgcn_cvt_pk_fp8_f32(xs, 0.f, 0, false);
-        const float r = xs - __builtin_amdgcn_cvt_f32_fp8(q1, 0);  // exact
-        p1 = (uint32_t)q1 & 0xffu;
-        p2 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(r, 0.f, 0, false) & 0xffu;
-      }
-      w1[i / 4] |= p1 << (8 * (i & 3));
-      w2[i / 4] |= p2 << (8 * (i & 3));
-    }
-    const int m0 = 2 * t, m1 = 2 * t + 1;
-    *reinterpret_cast<uint4*>(ch + m0 * 256 + ((c ^ (m0 & 15)) << 4)) =
-        make_uint4(w1[0], w1[1], w1[2], w1[3]);
-    *reinterpret_cast<uint4*>(ch + m1 * 256 + ((c ^ (m1 & 15)) << 4)) =
-        make_uint4(w2[0], w2[1], w2[2], w2[3]);
-    if (c == 0) {
-      ch[512 * M + t] = (uint8_t)e8;
-      reinterpret_cast<float*>(ch + 512 * M + 16)[t] = sum;
-    }
+    prep_token(v0, v1, live, c, t, M, ws + ((int64_t)d * max_stages + s) * pl_chunk(M));
   }
 }
 
@@ -841,13 +893,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_pl_kernel(const plz_gemv_desc
     }
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
-      // the row's palette entries as fp32 (bf16 bits: high byte from hi, low byte from lo)
-      const uint32_t lo = lr[u][r].x, hi = lr[u][r].y;
-      const float p0 = __uint_as_float(perm(hi, lo, 0x04000c0cu));
-      const float p1 = __uint_as_float(perm(hi, lo, 0x05010c0cu));
-      const float p2 = __uint_as_float(perm(hi, lo, 0x06020c0cu));
-      const float p3 = __uint_as_float(perm(hi, lo, 0x07030c0cu));
-      const float c1 = p1 - p0, c2 = p2 - p0, c3 = (p3 - p2) - c1;
+      float p0, c1, c2, c3;
+      plane_coefs(lr[u][r].x, lr[u][r].y, p0, c1, c2, c3);
       const uint4 wv = wr[u][r];
       const uint32_t wq[4] = {wv.x, wv.y, wv.z, wv.w};
       f32x4 cb0[NSET], cb1[NSET], cb3[NSET];
@@ -986,6 +1033,237 @@ __global__ void pack_planes_kernel(const uint32_t* __restrict__ packed, uint4* _
   out[t] = v;
 }
 
+// ---- bit planes, small launches: the reduction split over a workgroup's waves ----------------
+// A launch of few items (one layer's q/k/v, o, gate/up or down) leaves gemv_pl_kernel with one
+// 4-wave workgroup on some of the CUs, each walking all of K alone behind the prep launch: it is
+// bound by those serial chains, not by bandwidth. The split kernel gives a workgroup 16 * RBW rows
+// of one linear and spreads its stages over its waves; each wave leaves its partial sums in LDS, and
+// the same workgroup folds them in stage order, with the very operations of gemv_pl_kernel, so a
+// linear's outputs have the same bits whichever kernel a launch takes. Measured (hipGraph, weights
+// from HBM, prep + GEMV before -> one launch after, M = 1 / 4 / 8): one layer's q/k/v
+// 13.2 / 17.7 / 18.0 -> 6.0 / 6.7 / 8.0 us, o 17.2 / 22.4 / 23.2 -> 5.8 / 6.7 / 9.3, gate/up
+// 13.5 / 18.6 / 19.3 -> 10.4 / 14.2 / 18.2, down 26.1 / 31.6 / 33.9 -> 10.9 / 12.8 / 17.1. (The
+// decode layout chains its MFMAs through one accumulator over all of K: splitting that needs
+// per-chunk sums in the streaming kernel too, which cost it 1.3% at M = 16.)
+constexpr int SP_WAVES = 16;  // most waves per workgroup
+// This workgroup's linear and its first row. Descriptors of up to 64 linears are searched with
+// one load per lane and a ballot (a binary search would chain its loads).
+template <bool GROUPED>
+__device__ __forceinline__ plz_gemv_desc split_desc(const Table<GROUPED>& tb, int rows_per_wg,
+                                                    int64_t& row0) {
+  const int per_item = ROWS / rows_per_wg;
+  const int64_t item = blockIdx.x / per_item;
+  int di = 0;
+  if (GROUPED) {
+    if (tb.n <= 64) {
+      const int lane = threadIdx.x & 63;
+      const bool le = lane < tb.n && tb.descs[lane < tb.n ? lane : 0].block_begin <= item;
+      di = 63 - __builtin_clzll(__ballot(le));  // descriptor 0 begins at item 0
+    } else {
+      di = tb.find_item(item);
+    }
+    di = __builtin_amdgcn_readfirstlane(di);
+  }
+  const plz_gemv_desc d = tb.at(di);
+  row0 = (item - d.block_begin) * ROWS + (int64_t)(blockIdx.x % per_item) * rows_per_wg;
+  return d;
+}
+
+// Bit planes (M <= 8), one stage per wave and pass. The workgroup makes a pass's x pieces itself,
+// in LDS (16 lanes per token and stage: gemv_pl_prep_kernel's values without its launch), two
+// buffers of them so that a pass's pieces are made beside the MFMAs of the one before. A wave
+// leaves the plane sums S(b0), S(b1), S(b0 b1) of every C element in LDS [wave][row block]
+// [plane][element pair][lane]; the fold runs gemv_pl_kernel's chain of fma over the stages in
+// order, one thread per two C elements (a token's two pieces). NI: C rows per lane that hold a
+// token's piece (2 at M = 1). Every lane stores its elements, also those that hold no token: a
+// lane condition around the stores would let the compiler sink the MFMAs into it, where the
+// masked-off lanes' operands are missing.
+template <int NI>
+__host__ __device__ constexpr int sp_sum_bytes(int rbw) {  // plane sums and lookup words, a wave
+  return rbw * (3 * NI * 64 * 4 + 16 * 8);
+}
+template <int NI>
+__host__ __device__ constexpr int sp_wave_bytes(int rbw, int M) {
+  return sp_sum_bytes<NI>(rbw) + 2 * pl_chunk(M);
+}
+template <int NI, int RBW, bool GROUPED>
+__global__ __launch_bounds__(64 * SP_WAVES) void gemv_pl_split_kernel(
+    const plz_gemv_desc* __restrict__ descs, int n_desc, plz_gemv_desc single, int M) {
+  extern __shared__ uint4 smem[];
+  constexpr int NP = NI / 2, SB = sp_sum_bytes<NI>(RBW), LUT_OFF = RBW * 3 * NI * 64 * 4;
+  const Table<GROUPED> tb{descs, n_desc, single};
+  int64_t row0;
+  const plz_gemv_desc d = split_desc<GROUPED>(tb, 16 * RBW, row0);
+  if (row0 >= d.N) return;  // uniform: the item's rows past N
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nw = blockDim.x >> 6;
+  const int nl = lane & 15, q = lane >> 4;
+  const int m = nl < 2 * M ? nl : 2 * M - 1;  // A row of this lane (rows past 2M repeat one)
+  const int stages = (int)(d.K / KC), CH = pl_chunk(M);
+  const int64_t item0 = row0 / ROWS * ROWS;
+  const int blk0 = (int)(row0 - item0) / 16;
+  const uint4* words = reinterpret_cast<const uint4*>(
+      reinterpret_cast<const uint8_t*>(d.packed_items) + item0 * (d.K / 4)) + blk0 * 64 + lane;
+  const uint2* luts = reinterpret_cast<const uint2*>(
+      reinterpret_cast<const uint8_t*>(d.palette_items) + item0 * (d.K / kPalGroup) * 8) +
+      16 * blk0 + nl;
+  uint8_t* const sums = reinterpret_cast<uint8_t*>(smem);  // [nw][SB]
+  uint8_t* const xbuf = sums + nw * SB;                    // [2][nw][CH]
+  constexpr int kScale1 = 127, kScale2 = 128, kScaleH = 126;
+  constexpr uint32_t M1 = 0x11111111u, M2 = 0x22222222u, M4 = 0x44444444u;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+
+  // x pieces of stages s0 .. s0 + nw - 1 into buffer b
+  auto prep = [&](int s0, int b) {
+    const int work = (stages - s0 < nw ? stages - s0 : nw) * M, c = threadIdx.x & 15;
+    for (int w0 = 0; w0 < work; w0 += 4 * nw) {
+      const int w = w0 + ((int)threadIdx.x >> 4);
+      const bool live = w < work;
+      const int u = live ? w / M : 0, t = live ? w % M : 0;
+      const uint4* src = reinterpret_cast<const uint4*>(
+          d.x + (int64_t)t * d.K + (int64_t)(s0 + u) * KC + prep_k(c));
+      prep_token(src[0], src[1], live, c, t, M, xbuf + (b * nw + u) * CH);
+    }
+  };
+  uint4 wn[RBW];  // the wave's next stage, loaded a pass ahead
+  uint2 ln[RBW];
+  auto load = [&](int s) {
+#pragma unroll
+    for (int r = 0; r < RBW; ++r) {
+      wn[r] = words[(int64_t)s * (W_BYTES / 16) + r * 64];
+      ln[r] = luts[(int64_t)s * ROWS + r * 16];
+    }
+  };
+
+  // fold thread (row block fr, element pair fi, lane fl): C rows 4 (fl / 16) + 2 fi, + 1 = the
+  // two pieces of token 2 (fl / 16) + fi, column fl % 16
+  const int fl = lane, fi = (threadIdx.x >> 6) % NP, fr = (threadIdx.x >> 6) / NP;
+  const int tok = 2 * (fl >> 4) + fi;
+  const bool folds = fr < RBW && tok < M;
+  float y0 = 0.f, y1 = 0.f;
+
+  if (wave < stages) load(wave);
+  prep(0, 0);
+  __syncthreads();
+  for (int s0 = 0, b = 0; s0 < stages; s0 += nw, b ^= 1) {
+    if (s0 + wave < stages) {
+      uint4 wv[RBW];
+      uint2 lv[RBW];
+#pragma unroll
+      for (int r = 0; r < RBW; ++r) { wv[r] = wn[r]; lv[r] = ln[r]; }
+      if (s0 + nw + wave < stages) load(s0 + nw + wave);
+      const uint8_t* xs = xbuf + (b * nw + wave) * CH;
+      const int sc = xs[512 * M + (m >> 1)];
+      i32x8 a[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int c0 = 8 * h + 2 * q;
+        const uint4 lo = *reinterpret_cast<const uint4*>(xs + m * 256 + ((c0 ^ (m & 15)) << 4));
+        const uint4 hi = *reinterpret_cast<const uint4*>(xs + m * 256 + (((c0 + 1) ^ (m & 15)) << 4));
+        a[h] = i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w,
+                     (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+      }
+      uint8_t* st = sums + wave * SB;
+#pragma unroll
+      for (int r = 0; r < RBW; ++r) {
+        const uint32_t wq[4] = {wv[r].x, wv[r].y, wv[r].z, wv[r].w};
+        f32x4 cb[3] = {zero, zero, zero};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t m0 = h ? M4 : M1, m1 = h ? M4 : M2;
+          i32x8 B0 = {0, 0, 0, 0, 0, 0, 0, 0}, B1 = B0, B3 = B0;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t tj = wq[j] >> 1;
+            B0[j] = (int)(wq[j] & m0);
+            B1[j] = (int)((h ? tj : wq[j]) & m1);
+            B3[j] = (int)(wq[j] & tj & m0);
+          }
+          const int s02 = h ? kScaleH : kScale2, s1 = h ? kScaleH : kScale1;
+          cb[0] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[h], B0, cb[0], 0, 4, 0, sc, 0, s02);
+          cb[1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[h], B1, cb[1], 0, 4, 0, sc, 0, s1);
+          cb[2] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[h], B3, cb[2], 0, 4, 0, sc, 0, s02);
+        }
+        float2* dst = reinterpret_cast<float2*>(st) + r * 3 * NP * 64;
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+#pragma unroll
+          for (int i = 0; i < NP; ++i)
+            dst[(p * NP + i) * 64 + lane] = make_float2(cb[p][2 * i], cb[p][2 * i + 1]);
+        // the row's lookup words, the same from its four lanes
+        reinterpret_cast<uint2*>(st + LUT_OFF)[16 * r + nl] = lv[r];
+      }
+    }
+    if (s0 + nw < stages) prep(s0 + nw, b ^ 1);
+    __syncthreads();
+    const int ns = stages - s0 < nw ? stages - s0 : nw;
+    if (folds)
+      for (int u = 0; u < ns; ++u) {
+        const uint8_t* st = sums + u * SB;
+        const float2* src = reinterpret_cast<const float2*>(st) + (fr * 3 * NP + fi) * 64 + fl;
+        const float2 b0 = src[0], b1 = src[NP * 64], b3 = src[2 * NP * 64];
+        const uint2 lut = reinterpret_cast<const uint2*>(st + LUT_OFF)[16 * fr + (fl & 15)];
+        const float xs = reinterpret_cast<const float*>(xbuf + (b * nw + u) * CH + 512 * M + 16)[tok];
+        float p0, c1, c2, c3;
+        plane_coefs(lut.x, lut.y, p0, c1, c2, c3);
+        y0 = __builtin_fmaf(c1, b0.x, __builtin_fmaf(c2, b1.x, __builtin_fmaf(c3, b3.x, y0)));
+        y0 = __builtin_fmaf(p0, xs, y0);
+        y1 = __builtin_fmaf(c1, b0.y, __builtin_fmaf(c2, b1.y, __builtin_fmaf(c3, b3.y, y1)));
+      }
+    if (s0 + nw < stages) __syncthreads();  // the next pass overwrites the sums
+  }
+  const int64_t n = row0 + 16 * fr + (fl & 15);
+  if (folds && n < d.N) d.y[(int64_t)tok * d.N + n] = (uint16_t)f2bf(y0 + y1);
+}
+
+// Shape of a split launch: rbw row blocks (16 rows) per workgroup, 0 to stream, and its waves.
+struct SplitPlan {
+  int rbw, waves;
+};
+// most: the items (128 rows) up to which a split launch is the faster one; max_rbw: the kernel's
+// most row blocks; stages: of the longest linear, a wave takes one per pass.
+// Workgroups of 16 waves fill a CU at these register counts, so rbw is the least that leaves
+// one round of them, and a launch of more workgroups than CUs gets at most 8 waves each. Measured
+// on 2560 -> 9728 (76 items) at M = 1 / 4: 7.3 / 11.4 us in one round of 152 / 304 workgroups
+// of 10 waves, 8.1 / 9.2 us with 304 of 5.
+static SplitPlan split_plan(int64_t items, int64_t most, int max_rbw, int64_t stages) {
+  SplitPlan p{0, 0};
+  const int64_t cus = cu_count();
+  if (items > most) return p;
+  p.rbw = items * 8 <= cus ? 1 : items * 4 <= cus ? 2 : 4;
+  p.rbw = p.rbw < max_rbw ? p.rbw : max_rbw;
+  const int64_t cap = items * (8 / p.rbw) <= cus ? SP_WAVES : SP_WAVES / 2;
+  const int64_t passes = (stages + cap - 1) / cap;
+  p.waves = (int)((stages + passes - 1) / passes);
+  return p;
+}
+template <int NI, int RBW, bool GROUPED>
+static int launch_pl_split_r(int waves, int64_t items, hipStream_t st, const plz_gemv_desc* descs,
+                             int n, plz_gemv_desc single, int M, const char* what) {
+  auto kern = gemv_pl_split_kernel<NI, RBW, GROUPED>;
+  constexpr int kMost = 160 * 1024;
+  const int fit = kMost / sp_wave_bytes<NI>(RBW, M);
+  waves = waves < fit ? waves : fit;
+  waves = waves < RBW * NI / 2 ? RBW * NI / 2 : waves;  // the folds take RBW * NI / 2 waves
+  static_assert(RBW * NI / 2 * sp_wave_bytes<NI>(RBW, NI == 2 ? 1 : 8) <= kMost, "LDS");
+  static uint64_t lds_done = 0;
+  if (int rc = reserve_lds((const void*)kern, kMost, lds_done, what)) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(items * (8 / RBW))), dim3(64 * waves),
+                     (size_t)waves * sp_wave_bytes<NI>(RBW, M), st, descs, n, single, M);
+  return check_launch(what);
+}
+template <int NI, bool GROUPED>
+static int launch_pl_split(SplitPlan p, int64_t items, hipStream_t st, const plz_gemv_desc* descs,
+                           int n, plz_gemv_desc single, int M, const char* what) {
+  if constexpr (NI == 2)  // at M > 1 the plane sums of four row blocks leave LDS for too few waves
+    if (p.rbw == 4)
+      return launch_pl_split_r<NI, 4, GROUPED>(p.waves, items, st, descs, n, single, M, what);
+  if (p.rbw == 2)
+    return launch_pl_split_r<NI, 2, GROUPED>(p.waves, items, st, descs, n, single, M, what);
+  return launch_pl_split_r<NI, 1, GROUPED>(p.waves, items, st, descs, n, single, M, what);
+}
+
 template <int NX, int NSET, int NI, bool GROUPED>
 static int launch_pl_nx(int64_t items, hipStream_t st, const plz_gemv_desc* descs, int n,
                         plz_gemv_desc single, int M, int max_stages, uint8_t* ws,
@@ -1018,6 +1296,14 @@ template <bool GROUPED>
 static int launch_pl(int64_t items, hipStream_t st, const plz_gemv_desc* descs, int n,
                      plz_gemv_desc single, int M, int max_stages, uint8_t* ws, size_t ws_bytes,
                      const char* what) {
+  // up to one item per CU at M = 1 (240 items: 22.6 us against 27.9 streaming; 304 tie), where the
+  // x pieces are a sixteenth of the work; they are made once per workgroup, so from M = 2 up to
+  // 5/8 (152 items at M = 4 / 8: 14.0 / 18.0 us against 18.6 / 19.3; 240: 34 / 42 against 33 / 35)
+  const SplitPlan p =
+      split_plan(items, M == 1 ? cu_count() : cu_count() * 5 / 8, M == 1 ? 4 : 2, max_stages);
+  if (M <= 8 && p.rbw)
+    return M == 1 ? launch_pl_split<2, GROUPED>(p, items, st, descs, n, single, M, what)
+                  : launch_pl_split<4, GROUPED>(p, items, st, descs, n, single, M, what);
   if (M == 1)
     return launch_pl_nx<pl_nx(1), 1, 2, GROUPED>(items, st, descs, n, single, M, max_stages, ws,
                                                  ws_bytes, what);

@@ -371,3 +371,21 @@ def test_gemv_group_auto_layout(dev, M):
     assert grp.layout == (ops._lib.PLZ_GEMV_PLANES if M <= 8 else ops._lib.PLZ_GEMV_DECODE)
     for y, want in zip(grp.run(), wants):
         assert_close(f32(y), want, what=f"auto-layout gemv M={M}")
+
+
+@pytest.mark.parametrize("M", [1, 2, 7, 8])
+@pytest.mark.parametrize("N,K", [(8, 256), (136, 512), (264, 2560), (1024, 4352), (520, 9728)])
+def test_gemv_split_launch_is_the_streaming_launch_bit_for_bit(dev, M, N, K):
+    """A bit-plane launch of few items splits each linear's reduction over a workgroup's waves (edges: one
+    stage, one pass more than the waves hold, rows that end inside a row block); beside a linear
+    of 300 items the same linear is streamed. Both add in the same order."""
+    idx, pal = make_weight(N, K, seed=N + K)
+    x = randn_bf16(M, K, seed=M + K)
+    small = (x.to(dev), _packed(idx, dev), pal.to(dev))
+    idx2, pal2 = make_weight(128 * 300, 256, seed=1)
+    big = (randn_bf16(M, 256, seed=2).to(dev), _packed(idx2, dev), pal2.to(dev))
+    split = ops.GemvGroup([small], layout="planes").run()[0]
+    streamed = ops.GemvGroup([small, big], layout="planes").run()[0]
+    assert torch.equal(split, streamed)
+    assert_close(f32(split), O.lut_linear_fwd(f32(x), O.dequant(idx.numpy(), pal.numpy())),
+                 what=f"split gemv M={M} N={N} K={K}")
