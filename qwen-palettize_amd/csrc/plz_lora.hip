@@ -8,8 +8,8 @@
 // All four stream one M x L activation (x or grad_y) and touch a rank-r operand that stays in
 // L2, so they are HBM-bound: the work per activation element is r <= 32 MACs. Two kernels:
 //
-// rows_ring_kernel  (t, gt): a workgroup owns 64 rows of the activation and streams them
-//   through a 3-slot LDS ring of 256-element stages (whole 512-byte row segments per copy);
+// rows_ring_kernel  (t, gt): a workgroup owns 64 (or 16) rows of the activation and streams them
+//   through an LDS ring (3 slots, or up to 9) of 256-element stages (whole 512-byte row segments per copy);
 //   its 8 waves take one 32-wide 16x16x32 k-step of each stage and meet in LDS at the end.
 //   lora_a [r, L] is staged in the same row layout, lora_b [L, r] as its contiguous block.
 // cols_kernel  (grad_A, grad_B): the reduction index m is the activation's row, so fragments
@@ -54,8 +54,8 @@ __device__ __forceinline__ bf16x8 as_frag(uint4 v) { return __builtin_bit_cast(b
 //   BOP_T: Bop(l, j) = bop[j * L + l]  (lora_a, [r, L]);  else Bop(l, j) = bop[l * r + j]
 //   RG = 16-column groups (r <= 16 * RG)
 // The activation is staged through LDS. A workgroup owns
-// 64 rows; a stage is their next 256 reduction elements (32 KB) plus the matching slice of
-// Bop, copied global -> LDS by buffer_load ... lds into a 3-slot ring two stages ahead. Every
+// ROWS rows; a stage is their next 256 reduction elements (512 B a row) plus the matching slice of
+// Bop, copied global -> LDS by buffer_load ... lds into a ring, NS - 1 stages ahead. Every
 // copy instruction moves 1 KB of whole 512-byte row segments, so the stream reads whole cache
 // lines in order instead of 16 rows x 64 B per instruction (an 84 MB probe of the two
 // patterns: 15 against 18-19 us). The 8 waves split each stage's 256 elements (32 each: one
@@ -65,26 +65,35 @@ __device__ __forceinline__ bf16x8 as_frag(uint4 v) { return __builtin_bit_cast(b
 //   Bop (BOP_T, lora_a [r, L]): rows j of the same layout.
 //   Bop (else, lora_b [L, r]): the stage's contiguous [256][r] block as it is in memory.
 // ---------------------------------------------------------------------------------------
-constexpr int RR_ROWS = 64;                       // activation rows per workgroup
+// A workgroup owns ROWS activation rows. 64 (three ring slots) stream a large activation at its
+// bandwidth. With few rows a launch is a serial chain of L / 256 stages on few CUs, bound by the
+// latency of a stage's copies over the stages in flight: 16 rows make more workgroups and a stage
+// of 16-24 KB, of which RR_SLOTS = 9 or 6 fit in LDS.
 constexpr int RR_KC = 256;                        // reduction elements per stage
-constexpr int RR_NS = 3;                          // ring slots (copies two stages ahead)
-constexpr int RR_XBYTES = RR_ROWS * RR_KC * 2;    // 32 KB
-constexpr int RR_XI = RR_XBYTES / (512 * 16);     // X copies per thread per stage (4)
-template <int RG>
-constexpr int rr_stage_bytes() { return RR_XBYTES + RG * 8192; }  // + Bop: RG x 8 KB
+template <int ROWS>
+constexpr int rr_xbytes() { return ROWS * RR_KC * 2; }
+template <int ROWS, int RG>
+constexpr int rr_stage_bytes() { return rr_xbytes<ROWS>() + RG * 8192; }  // + Bop: RG x 8 KB
+template <int ROWS, int RG>
+constexpr int rr_slots() {  // ring slots (copies that many stages ahead, less one)
+  return ROWS == 64 ? 3 : 160 * 1024 / rr_stage_bytes<ROWS, RG>() < 9
+             ? 160 * 1024 / rr_stage_bytes<ROWS, RG>() : 9;
+}
 
-template <bool BOP_T, int RG>
+template <bool BOP_T, int RG, int ROWS>
 __global__ __launch_bounds__(512) void rows_ring_kernel(const uint16_t* __restrict__ X,
                                                         const uint16_t* __restrict__ bop,
                                                         uint16_t* __restrict__ out, float scale,
                                                         int64_t M, int L, int r) {
   extern __shared__ uint4 smem[];
   lds_u8* lds = (lds_u8*)smem;
-  constexpr int STAGE = rr_stage_bytes<RG>();
+  constexpr int STAGE = rr_stage_bytes<ROWS, RG>(), NS = rr_slots<ROWS, RG>();
+  constexpr int G = ROWS / 16, XI = ROWS / 16;  // row groups; X copies per thread and stage
+  constexpr int XBYTES = rr_xbytes<ROWS>();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int rr = lane & 15, q = lane >> 4;
-  const int64_t m0 = (int64_t)blockIdx.x * RR_ROWS;
-  const int rows = (int)min((int64_t)RR_ROWS, M - m0);
+  const int64_t m0 = (int64_t)blockIdx.x * ROWS;
+  const int rows = (int)min((int64_t)ROWS, M - m0);
   const int nst = (L + RR_KC - 1) / RR_KC;
   // rows past the end of X, and reduction indices past L, read as zero (range check or kBufOob)
   const BufRsrc xr = make_rsrc(X + m0 * L, (uint32_t)rows * (uint32_t)L * 2u);
@@ -96,11 +105,11 @@ __global__ __launch_bounds__(512) void rows_ring_kernel(const uint16_t* __restri
     const bool live = s < nst;
     const int k0 = RR_KC * s;
 #pragma unroll
-    for (int it = 0; it < RR_XI; ++it) {
-      const int p = (wave * RR_XI + it) * 64 + lane;  // physical chunk: row p / 32
+    for (int it = 0; it < XI; ++it) {
+      const int p = (wave * XI + it) * 64 + lane;  // physical chunk: row p / 32
       const int m = p >> 5, k = k0 + 8 * ((p & 31) ^ (m & 15));
       const uint32_t off = live && k < L ? ((uint32_t)m * (uint32_t)L + (uint32_t)k) * 2u : kBufOob;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_u8*)(ss + (wave * RR_XI + it) * 1024), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_u8*)(ss + (wave * XI + it) * 1024), 16,
                                                off, 0, 0, 0);
     }
 #pragma unroll
@@ -114,27 +123,27 @@ __global__ __launch_bounds__(512) void rows_ring_kernel(const uint16_t* __restri
         if (live && 8 * p < RR_KC * r) off = ((uint32_t)k0 * (uint32_t)r + 8u * p) * 2u;
       }
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          br, (lds_u8*)(ss + RR_XBYTES + (wave * RG + it) * 1024), 16, off, 0, 0, 0);
+          br, (lds_u8*)(ss + XBYTES + (wave * RG + it) * 1024), 16, off, 0, 0, 0);
     }
   };
 
-  f32x4 acc[4][RG];
+  f32x4 acc[G][RG];
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
+  for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int cg = 0; cg < RG; ++cg) acc[g][cg] = f32x4{0.f, 0.f, 0.f, 0.f};
   // lane (rr, q) of wave w: logical chunk 4w + q (reduction elements 32w + 8q .. +7 of the stage)
   const int c = 4 * wave + q;
   const int xoff = rr * 512 + ((c ^ rr) << 4);  // row rr of a group; (16g + rr) & 15 == rr
-  // the copies of stage s + RR_NS - 1 go to slot ws before the MFMAs read slot xs (distinct
+  // the copies of stage s + NS - 1 go to slot ws before the MFMAs read slot xs (distinct
   // slots: __restrict__ keeps the compiler from waiting on the new copies first)
   auto step = [&](int s, const lds_u8* __restrict__ xs, lds_u8* __restrict__ ws) {
-    issue(s + RR_NS - 1, ws);
-    bf16x8 a[4], b[RG];
+    issue(s + NS - 1, ws);
+    bf16x8 a[G], b[RG];
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+    for (int g = 0; g < G; ++g)
       a[g] = __builtin_bit_cast(bf16x8, *(const lds_w4*)(xs + g * 16 * 512 + xoff));
-    const lds_u8* bs = xs + RR_XBYTES;
+    const lds_u8* bs = xs + XBYTES;
 #pragma unroll
     for (int cg = 0; cg < RG; ++cg) {
       if constexpr (BOP_T) {
@@ -152,16 +161,16 @@ __global__ __launch_bounds__(512) void rows_ring_kernel(const uint16_t* __restri
       }
     }
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+    for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int cg = 0; cg < RG; ++cg) acc[g][cg] = mfma16(a[g], b[cg], acc[g][cg]);
   };
 #pragma unroll
-  for (int s = 0; s < RR_NS - 1; ++s) issue(s, lds + s * STAGE);
+  for (int s = 0; s < NS - 1; ++s) issue(s, lds + s * STAGE);
   for (int s = 0; s < nst; ++s) {
-    wait_vmcnt<(RR_XI + RG) * (RR_NS - 2)>();  // this lane's copies of stage s have landed
-    lds_barrier();                               // everyone's have; slot (s-1) % RR_NS is free
-    step(s, lds + (s % RR_NS) * STAGE, lds + ((s + RR_NS - 1) % RR_NS) * STAGE);
+    wait_vmcnt<(XI + RG) * (NS - 2)>();  // this lane's copies of stage s have landed
+    lds_barrier();                               // everyone's have; slot (s-1) % NS is free
+    step(s, lds + (s % NS) * STAGE, lds + ((s + NS - 1) % NS) * STAGE);
   }
   __builtin_amdgcn_s_waitcnt(0);  // drain the trailing (empty) copies
   lds_barrier();                  // the ring is free: the cross-wave sums reuse it
@@ -171,18 +180,18 @@ __global__ __launch_bounds__(512) void rows_ring_kernel(const uint16_t* __restri
   constexpr int RS = RG * 16 + 1;
   float* red = reinterpret_cast<float*>(smem);
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
+  for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int cg = 0; cg < RG; ++cg)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        red[(wave * RR_ROWS + 16 * g + 4 * q + e) * RS + 16 * cg + rr] = acc[g][cg][e];
+        red[(wave * ROWS + 16 * g + 4 * q + e) * RS + 16 * cg + rr] = acc[g][cg][e];
   __syncthreads();
   for (int idx = threadIdx.x; idx < rows * r; idx += 512) {
     const int row = idx / r, j = idx - row * r;
     float sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < 8; ++w) sum += red[(w * RR_ROWS + row) * RS + j];
+    for (int w = 0; w < 8; ++w) sum += red[(w * ROWS + row) * RS + j];
     out[(m0 + row) * r + j] = (uint16_t)f2bf(scale * sum);
   }
 }
@@ -487,24 +496,31 @@ static int cols(const uint16_t* x, const uint16_t* grad_y, const uint16_t* t, co
   return check_launch(what);
 }
 
+template <bool BOP_T, int RG, int ROWS>
+static int rows_launch(const uint16_t* X, const uint16_t* bop, float scale, uint16_t* out,
+                       int64_t M, int64_t L, int r, hipStream_t s, const char* what) {
+  auto kern = rows_ring_kernel<BOP_T, RG, ROWS>;
+  constexpr size_t lds = (size_t)rr_slots<ROWS, RG>() * rr_stage_bytes<ROWS, RG>();
+  static_assert(lds >= (size_t)8 * ROWS * (RG * 16 + 1) * 4, "the cross-wave sums reuse the ring");
+  static uint64_t done = 0;
+  if (int rc = reserve_lds((const void*)kern, lds, done, what)) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((M + ROWS - 1) / ROWS)), dim3(512), lds, s, X, bop, out,
+                     scale, M, (int)L, r);
+  return check_launch(what);
+}
+// 16 rows per workgroup while that is at most one workgroup per CU, else 64 (both add in the same
+// order: the same bits). Measured, 64 -> 16 rows: t at K 9728 / 2560, rank 32 / 16: M = 48
+// 21.2 / 6.4 -> 13.3 / 4.7 us, M = 1024 22.0 / 7.5 -> 14.0 / 5.2, M = 4096 37.4 / 8.0 -> 24.0 / 6.6;
+// gt at N 9728, M = 1024 / 4096: 22.0 / 32.8 -> 15.9 / 19.9. Above that the shared operand's
+// re-reads count: M = 16384 58.3 / 17.9 us with 64 rows, 85.1 / 25.1 with 16.
 template <bool BOP_T>
 static int rows(const uint16_t* X, const uint16_t* bop, float scale, uint16_t* out, int64_t M,
                 int64_t L, int r, hipStream_t s, const char* what) {
-  const dim3 grid((unsigned)((M + RR_ROWS - 1) / RR_ROWS));
-  static uint64_t done1 = 0, done2 = 0;
-  int rc;
-  if (r <= 16) {
-    constexpr size_t lds = (size_t)RR_NS * rr_stage_bytes<1>();
-    if ((rc = reserve_lds((const void*)rows_ring_kernel<BOP_T, 1>, lds, done1, what))) return rc;
-    hipLaunchKernelGGL((rows_ring_kernel<BOP_T, 1>), grid, dim3(512), lds, s, X, bop, out, scale,
-                       M, (int)L, r);
-  } else {
-    constexpr size_t lds = (size_t)RR_NS * rr_stage_bytes<2>();
-    if ((rc = reserve_lds((const void*)rows_ring_kernel<BOP_T, 2>, lds, done2, what))) return rc;
-    hipLaunchKernelGGL((rows_ring_kernel<BOP_T, 2>), grid, dim3(512), lds, s, X, bop, out, scale,
-                       M, (int)L, r);
-  }
-  return check_launch(what);
+  if (M <= 16 * (int64_t)cu_count())
+    return r <= 16 ? rows_launch<BOP_T, 1, 16>(X, bop, scale, out, M, L, r, s, what)
+                   : rows_launch<BOP_T, 2, 16>(X, bop, scale, out, M, L, r, s, what);
+  return r <= 16 ? rows_launch<BOP_T, 1, 64>(X, bop, scale, out, M, L, r, s, what)
+                 : rows_launch<BOP_T, 2, 64>(X, bop, scale, out, M, L, r, s, what);
 }
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -522,7 +538,7 @@ int plz_lora_project(const uint16_t* x, const uint16_t* lora_a, float scale, uin
   PLZ_REQUIRE(M >= 0 && K >= 0 && rank > 0 && rank <= 32 && rank % 8 == 0,
               "plz_lora_project: need M, K >= 0 and rank a multiple of 8 in [8, 32]");
   PLZ_REQUIRE(K % 8 == 0, "plz_lora_project: K must be a multiple of 8");
-  PLZ_REQUIRE(K < (1 << 24) && RR_ROWS * K * 2 < (int64_t)1 << 31,
+  PLZ_REQUIRE(K < (1 << 24) && 64 * K * 2 < (int64_t)1 << 31,
               "plz_lora_project: K (%lld) too large", (long long)K);
   if (M == 0) return PLZ_OK;
   PLZ_REQUIRE(x && lora_a && t && aligned16(x) && aligned16(lora_a),
@@ -535,7 +551,7 @@ int plz_lora_grad_t(const uint16_t* grad_y, const uint16_t* lora_b, float scale,
   PLZ_REQUIRE(M >= 0 && N >= 0 && rank > 0 && rank <= 32 && rank % 8 == 0,
               "plz_lora_grad_t: need M, N >= 0 and rank a multiple of 8 in [8, 32]");
   PLZ_REQUIRE(N % 8 == 0, "plz_lora_grad_t: N must be a multiple of 8");
-  PLZ_REQUIRE(N < (1 << 24) && RR_ROWS * N * 2 < (int64_t)1 << 31,
+  PLZ_REQUIRE(N < (1 << 24) && 64 * N * 2 < (int64_t)1 << 31,
               "plz_lora_grad_t: N (%lld) too large", (long long)N);
   if (M == 0) return PLZ_OK;
   PLZ_REQUIRE(grad_y && lora_b && gt && aligned16(grad_y) && aligned16(lora_b),

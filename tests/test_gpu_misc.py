@@ -28,6 +28,20 @@ def test_lora_project_and_grad_t(dev, M, L, rank):
     assert_close(f32(gt), 2.0 * (f32(x).astype(np.float64) @ f32(b)), what="lora gt")
 
 
+@pytest.mark.parametrize("L,rank", [(8, 8), (264, 16), (2560, 32), (4104, 24)])
+def test_lora_row_products_of_few_rows_bit_for_bit(dev, L, rank):
+    """16 rows per workgroup up to one workgroup per CU, 64 above: the same sums in the same
+    order (rings longer than the reduction, rows past the last block)."""
+    big = 16 * torch.cuda.get_device_properties(0).multi_processor_count + 1
+    x = randn_bf16(big, L, seed=L).to(dev)
+    a = randn_bf16(rank, L, seed=1, std=0.05).to(dev)
+    b = randn_bf16(L, rank, seed=2, std=0.05).to(dev)
+    t, gt = ops.lora_project(x, a, 0.5), ops.lora_grad_t(x, b, 2.0)
+    for M in (1, 15, 17, 100, big - 1):
+        assert torch.equal(ops.lora_project(x[:M].contiguous(), a, 0.5), t[:M]), M
+        assert torch.equal(ops.lora_grad_t(x[:M].contiguous(), b, 2.0), gt[:M]), M
+
+
 @pytest.mark.parametrize("M,N,K,rank", [(1000, 264, 512, 16), (1000, 264, 512, 32),
                                         (1, 8, 8, 8), (77, 520, 264, 24),
                                         (16384, 9728, 2560, 16), (16384, 2560, 9728, 32)])
