@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "plz_gemm2.cuh"
+#include "plz_skinny.h"
 #include "palettize_hip.h"
 
 namespace plz {
@@ -1126,7 +1127,9 @@ __global__ __launch_bounds__(NTHR) void gemm2_kernel(const Args g) {
       float4* dst = reinterpret_cast<float4*>(g.tail_ws) +
                     ((int64_t)(bid - g.tail_first) * g.tail_split + part) * (TILE * TILE / 4);
 #pragma unroll
-      for (int ti = 0; ti < WT_I; ++ti)
+      for (int ti = 0; ti < WT_I; ++ti) {
+        // blocks of rows or columns past the edge are never stored: no partials for them
+        if (i0 + wi * (32 * WT_I) + 32 * ti >= g.I || j0 + wj * (32 * WT_J) >= g.J) break;
 #pragma unroll
         for (int tj = 0; tj < WT_J; ++tj)
 #pragma unroll
@@ -1134,6 +1137,7 @@ __global__ __launch_bounds__(NTHR) void gemm2_kernel(const Args g) {
             dst[((ti * WT_J + tj) * 4 + e4) * NTHR + threadIdx.x] =
                 make_float4(acc[ti][tj][4 * e4], acc[ti][tj][4 * e4 + 1],
                             acc[ti][tj][4 * e4 + 2], acc[ti][tj][4 * e4 + 3]);
+      }
       return;
     }
     store_tile_bf16(g, acc, lbase, i0, j0, wi, wj, lane);
@@ -1330,6 +1334,10 @@ __global__ __launch_bounds__(TAIL_THREADS) void tail_reduce_kernel(const Args g)
   const int wj = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const float4* src = reinterpret_cast<const float4*>(g.tail_ws) +
                       (int64_t)tt * g.tail_split * (TILE * TILE / 4);
+  // the slab's rows and this wave's columns past the edge have no partials (and are not stored)
+  const int64_t i0 = (int64_t)tile_i * TILE + (TILE / TAIL_SLABS) * q, j0 = (int64_t)tile_j * TILE;
+  if (i0 >= g.I) return;
+  const int live = j0 + wj * (32 * WT_J) >= g.J ? 0 : i0 + 32 >= g.I ? 1 : 2;  // 32-row blocks
   float a[2][WT_J][16];
 #pragma unroll
   for (int tl = 0; tl < 2; ++tl)
@@ -1339,7 +1347,8 @@ __global__ __launch_bounds__(TAIL_THREADS) void tail_reduce_kernel(const Args g)
       for (int e = 0; e < 16; ++e) a[tl][tj][e] = 0.f;
   for (int p = 0; p < g.tail_split; ++p) {
 #pragma unroll
-    for (int tl = 0; tl < 2; ++tl)
+    for (int tl = 0; tl < 2; ++tl) {
+      if (tl >= live) break;
 #pragma unroll
       for (int tj = 0; tj < WT_J; ++tj)
 #pragma unroll
@@ -1351,9 +1360,9 @@ __global__ __launch_bounds__(TAIL_THREADS) void tail_reduce_kernel(const Args g)
           a[tl][tj][4 * e4 + 2] += v.z;
           a[tl][tj][4 * e4 + 3] += v.w;
         }
+    }
   }
   // bf16 (alpha * acc + bias) of the slab's 64 rows in LDS, as stage_tile_bf16 computes it
-  const int64_t i0 = (int64_t)tile_i * TILE + (TILE / TAIL_SLABS) * q, j0 = (int64_t)tile_j * TILE;
 #pragma unroll
   for (int tj = 0; tj < WT_J; ++tj) {
     const int col = wj * (32 * WT_J) + 32 * tj + (lane & 31);
@@ -1648,6 +1657,14 @@ constexpr int64_t kStagedRows = 4096;
 // 2, 6) 1085-1092 TFLOP/s against 1081 for 8, 1067-1069 for 16, 1053 for a column walk.
 constexpr int kDenseGroup = 4;
 
+// Up to 64 rows the forward runs the kernel of plz_skinny.hip: M = 17 / 48 / 64 in us against the
+// split 256-row tiles 2560 -> 4096 6.7 / 10.9 / 13.0 (24.0 / 34.7 / 34.8), 2560 -> 9728
+// 11.3 / 17.2 / 18.5 (27.8 / 37.8 / 37.8), 9728 -> 2560 17.5 / 32.6 / 41.0 (32.0 / 61.4 / 61.5). Its
+// time grows with M; at 128 rows 9728 -> 2560 is the slower one (80 against 65).
+static bool skinny_fwd_rows(int64_t M, int64_t K) {
+  return K > 0 && M <= sk::kMaxRows && M * K < ((int64_t)1 << 31);
+}
+
 static size_t staged_w_bytes(int64_t N, int64_t K) {
   return ((size_t)N * (size_t)K * sizeof(uint16_t) + 255) & ~(size_t)255;
 }
@@ -1675,7 +1692,7 @@ static bool stage_w(Args& g, const int32_t* packed, const float* palette, int64_
 extern "C" {
 
 size_t plz_lut_linear_fwd_workspace(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || skinny_fwd_rows(M, K)) return 0;
   if (M >= kStagedRows) return staged_w_bytes(N, K) + tail_bytes(M, N, K);
   return tail_bytes(M, N, K);
 }
@@ -1695,6 +1712,9 @@ int plz_lut_linear_fwd(const uint16_t* x, const int32_t* packed, const float* pa
               "plz_lut_linear_fwd: x, packed and palette must be 16-byte aligned");
   PLZ_REQUIRE(rank == 0 || (lora_t && lora_b && a16(lora_t) && a16(lora_b)),
               "plz_lut_linear_fwd: rank > 0 needs 16-byte aligned lora_t and lora_b");
+  if (skinny_fwd_rows(M, K))
+    return sk::fwd(x, packed, palette, bias, lora_t, lora_b, rank, y, M, N, K, cu_count(),
+                   (hipStream_t)stream, "plz_lut_linear_fwd");
   Args g = {};
   g.a = x; g.lda = K;
   g.I = M; g.J = N; g.R = K;

@@ -389,3 +389,38 @@ def test_gemv_split_launch_is_the_streaming_launch_bit_for_bit(dev, M, N, K):
     assert torch.equal(split, streamed)
     assert_close(f32(split), O.lut_linear_fwd(f32(x), O.dequant(idx.numpy(), pal.numpy())),
                  what=f"split gemv M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 64, 65])
+@pytest.mark.parametrize("N,K,rank,bias", [(8, 256, 0, True), (136, 768, 8, False),
+                                           (1000, 2304, 40, True), (4104, 256, 32, False),
+                                           (8200, 512, 64, True)])
+def test_lut_linear_fwd_few_rows(dev, M, N, K, rank, bias):
+    """The forward's kernel for up to 64 rows (one to four 16-row blocks of W per workgroup, by N;
+    one to four blocks of tokens; units of 128 k over eight waves; ranks past one 32-wide step)
+    and the first size past it."""
+    idx, pal, x, W, (a, b) = _oracle_problem(M, N, K, seed=M + N, rank=max(rank, 8))
+    bv = randn_bf16(N, seed=3, std=0.1) if bias else None
+    t = randn_bf16(M, rank, seed=5, std=0.1).to(dev) if rank else None
+    lb = randn_bf16(N, rank, seed=6, std=0.1).to(dev) if rank else None
+    y = ops.lut_linear_fwd(x.to(dev), _packed(idx, dev), pal.to(dev),
+                           bv.to(dev) if bias else None, t, lb)
+    want = O.lut_linear_fwd(f32(x), W, f32(bv) if bias else None)
+    if rank:
+        want = want + f32(t) @ f32(lb).T
+    assert_close(f32(y), want, what=f"few-row fwd M={M} N={N} K={K} rank={rank}")
+
+
+@pytest.mark.parametrize("M", [96, 300])
+def test_tail_parts_past_the_edge(dev, M):
+    """Split tiles whose last rows and columns lie past the matrix (no partials are kept for
+    those blocks): a ragged M below and above one tile, N inside a tile's first 64 columns."""
+    N, K = 1064, 2560
+    idx, pal, x, W, (a, b) = _oracle_problem(M, N, K, seed=M, rank=16)
+    assert ops.query("plz_lut_linear_fwd_workspace", M, N, K) > 0
+    p, pl = _packed(idx, dev), pal.to(dev)
+    assert_close(f32(ops.lut_linear_fwd(x.to(dev), p, pl)), O.lut_linear_fwd(f32(x), W),
+                 what="fwd")
+    gy = randn_bf16(M, N, seed=4)
+    assert_close(f32(ops.lut_linear_bwd_x(gy.to(dev), p, pl)), O.grad_x(f32(gy), W),
+                 what="grad_x")
