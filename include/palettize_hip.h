@@ -180,6 +180,12 @@ int plz_linear_fwd_dense_swiglu(const uint16_t* x, const uint16_t* w_gate_up, ui
 int plz_linear_fwd_dense_swiglu_cat(const uint16_t* x, const uint16_t* w, const uint16_t* lora_t,
                                     const uint16_t* lora_b, int rank, uint16_t* y, uint16_t* h,
                                     int64_t M, int64_t F, int64_t K, void* stream);
+/* y = x w (+ bias) for a weight stored [K, N]; the workspace is
+ * plz_linear_bwd_x_dense_workspace(M, K, N). */
+int plz_linear_fwd_dense_kn(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y,
+                            void* workspace, size_t workspace_bytes, int64_t M, int64_t N,
+                            int64_t K, void* stream);
+
 /* grad_x = grad_y w (+lora). Replaces torch.matmul(grad_y, W.T)
  * (fused_lut_linear_cuda.py:944). */
 int plz_linear_bwd_x_dense(const uint16_t* grad_y, const uint16_t* w, const uint16_t* lora_gt,
@@ -240,6 +246,25 @@ int64_t plz_pw_ref_plan(plz_pw_ref_desc* descs, int n, int64_t group_size);
 /* descs_device: a device copy of the planned descriptors. */
 int plz_soft_pw_ref_batched(const plz_pw_ref_desc* descs_device, int n, int64_t total_blocks,
                             int64_t group_size, float tau, uint32_t step_seed, void* stream);
+
+/* The soft linear in the reference's own layouts (fused_lut_kernel.cu:1946-2004, 1877-1924;
+ * triton_soft_forward.py:83-181): logits (4, K, N) bf16 / fp16, palette (G, 4) bf16 / fp16 / fp32
+ * with column n in group n / group_size, the LCG noise of `seed` (the CUDA hash, or with
+ * triton_hash the Triton one; idx = (k*N + n)*4 + c). K and N multiples of 8.
+ * build_w: w [K, N] bf16 per mode (PLZ_W_*); y = x w is plz_linear_fwd_dense_kn, grad_x =
+ * grad_y w^T plz_linear_fwd_dense(grad_y, w) with N and K exchanged.
+ * bwd: grad_logits (4, K, N) in the logits' type (may be null) and grad_palette (n_groups, 4) in
+ * the palette's type, for dW = grad_y^T x with x [M, K], grad_y [M, N]. */
+int plz_soft_ref_build_w(const uint16_t* logits, int logits_dtype, const void* palette,
+                         int palette_dtype, int64_t group_size, int triton_hash, uint32_t seed,
+                         float tau, int mode, uint16_t* w, int64_t K, int64_t N, void* stream);
+size_t plz_soft_ref_bwd_workspace(int64_t M, int64_t N, int64_t K);
+int plz_soft_ref_bwd(const uint16_t* x, const uint16_t* grad_y, const uint16_t* logits,
+                     int logits_dtype, const void* palette, int palette_dtype, int64_t n_groups,
+                     int64_t group_size, int triton_hash, uint32_t seed, float tau,
+                     int scale_grad_by_inv_tau, uint16_t* grad_logits, void* grad_palette,
+                     void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
+                     void* stream);
 
 /* Builds the forward weight of the soft path from logits [N, K, 4] (bf16 or fp16),
  * noise fp32 [N, K, 4] and palette fp32 [N, K/256, 4]:

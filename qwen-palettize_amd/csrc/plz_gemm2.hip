@@ -12,6 +12,7 @@
 
 #include "plz_gemm2.cuh"
 #include "plz_skinny.h"
+#include "plz_soft_ref.h"
 #include "palettize_hip.h"
 
 namespace plz {
@@ -1286,7 +1287,8 @@ __global__ __launch_bounds__(NTHR) void gemm2_kernel(const Args g) {
           const float2 gw =
               *reinterpret_cast<const float2*>(&sC[ptile(item >> 1, 128 * (item & 1) + 2 * lane)]);
           // this split's partial dW rows, [split][N][K] fp32
-          *reinterpret_cast<float2*>(g.acc_ws + ((int64_t)zsl * g.I + n) * g.J + kseg + 2 * lane) = gw;
+          if (kseg + 2 * lane < g.J)
+            *reinterpret_cast<float2*>(g.acc_ws + ((int64_t)zsl * g.I + n) * g.J + kseg + 2 * lane) = gw;
         }
       }
       if (wgrad && threadIdx.x >= 256)
@@ -1636,6 +1638,35 @@ static int pal_scratch(float** out) {
   }
   *out = reinterpret_cast<float*>(pal_scratch_addr[dev]);
   return PLZ_OK;
+}
+
+// Splits of R for dw_partials: (waves of tiles * z workgroups) x (stages per split + 4 of prologue
+// and epilogue) at 1.9 us, plus 8 B per element and split of partials written and read at 5 TB/s.
+int dw_splits(int64_t I, int64_t J, int64_t R) {
+  const int64_t tiles = ((I + TILE - 1) / TILE) * ((J + TILE - 1) / TILE), C = cu_count();
+  int best = 1;
+  double best_t = 1e300;
+  for (int z = 1; z <= 16; ++z) {
+    const int64_t len = split_len(R, z);
+    if (z > 1 && (len < 8 * BK || (int64_t)(z - 1) * len >= R)) break;  // >= 8 stages, none empty
+    const double t = (double)((tiles * z + C - 1) / C) * ((double)len / BK + 4.0) * 1.9 +
+                     z * 8.0 * (double)I * (double)J / 5.0e6;
+    if (t < best_t * 0.97) {
+      best_t = t;
+      best = z;
+    }
+  }
+  return best;
+}
+int dw_partials(const uint16_t* a, const uint16_t* b, float* out, int z, int64_t I, int64_t J,
+                int64_t R, hipStream_t stream, const char* what) {
+  Args g = {};
+  g.a = a; g.lda = I;
+  g.b = b; g.ldb = J;
+  g.I = I; g.J = J; g.R = R; g.r_split = split_len(R, z);
+  g.acc_ws = out;
+  g.group = J > I ? -1 : 1;  // walk the larger operand's panels, as the hard grad_palette GEMM
+  return launch<OP_COL, OP_COL, EPI_F32>(g, z, stream, what);
 }
 
 static size_t soft_pal_bytes(int64_t N, int64_t K) { return (size_t)N * (K / 128) * 4 * sizeof(float); }
@@ -2005,7 +2036,7 @@ size_t plz_linear_bwd_x_dense_workspace(int64_t M, int64_t N, int64_t K) {
 
 static int linear_bwd_x_dense(const uint16_t* grad_y, const uint16_t* w, const uint16_t* lora_gt,
                               const uint16_t* lora_a, int rank, const uint16_t* sw_pre,
-                              uint16_t* grad_x, void* workspace, size_t workspace_bytes, int64_t M,
+                              const uint16_t* bias, uint16_t* grad_x, void* workspace, size_t workspace_bytes, int64_t M,
                               int64_t N, int64_t K, void* stream, const char* what) {
   PLZ_REQUIRE(M >= 0 && N >= 0 && K >= 0, "%s: negative shape", what);
   PLZ_REQUIRE(K % 8 == 0 && N % 8 == 0, "%s: K and N must be multiples of 8", what);
@@ -2022,6 +2053,7 @@ static int linear_bwd_x_dense(const uint16_t* grad_y, const uint16_t* w, const u
   g.I = M; g.J = K; g.R = N;
   g.a2 = lora_gt; g.b2 = lora_a; g.R2 = rank;
   g.c = grad_x; g.ldc = sw_pre ? 2 * K : K; g.alpha = 1.f;
+  g.bias = bias;
   g.sw_pre = sw_pre; g.ld_sw = 2 * K;
   g.group = kDenseGroup;
   const int rc = set_tail(g, workspace, workspace_bytes, what);
@@ -2033,8 +2065,15 @@ int plz_linear_bwd_x_dense(const uint16_t* grad_y, const uint16_t* w, const uint
                            const uint16_t* lora_a, int rank, uint16_t* grad_x, void* workspace,
                            size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
                            void* stream) {
-  return linear_bwd_x_dense(grad_y, w, lora_gt, lora_a, rank, nullptr, grad_x, workspace,
+  return linear_bwd_x_dense(grad_y, w, lora_gt, lora_a, rank, nullptr, nullptr, grad_x, workspace,
                             workspace_bytes, M, N, K, stream, "plz_linear_bwd_x_dense");
+}
+
+int plz_linear_fwd_dense_kn(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y,
+                            void* workspace, size_t workspace_bytes, int64_t M, int64_t N,
+                            int64_t K, void* stream) {
+  return linear_bwd_x_dense(x, w, nullptr, nullptr, 0, nullptr, bias, y, workspace,
+                            workspace_bytes, M, K, N, stream, "plz_linear_fwd_dense_kn");
 }
 
 int plz_linear_bwd_x_dense_swiglu(const uint16_t* grad_y, const uint16_t* w,
@@ -2045,8 +2084,8 @@ int plz_linear_bwd_x_dense_swiglu(const uint16_t* grad_y, const uint16_t* w,
   PLZ_REQUIRE(M == 0 || K == 0 || (gate_up && grad_gate_up && a16(gate_up) && a16(grad_gate_up)),
               "plz_linear_bwd_x_dense_swiglu: gate_up and grad_gate_up must be non-null, "
               "16-byte aligned");
-  return linear_bwd_x_dense(grad_y, w, lora_gt, lora_a, rank, gate_up, grad_gate_up, workspace,
-                            workspace_bytes, M, N, K, stream, "plz_linear_bwd_x_dense_swiglu");
+  return linear_bwd_x_dense(grad_y, w, lora_gt, lora_a, rank, gate_up, nullptr, grad_gate_up,
+                            workspace, workspace_bytes, M, N, K, stream, "plz_linear_bwd_x_dense_swiglu");
 }
 
 size_t plz_soft_bwd_workspace(int64_t M, int64_t N, int64_t K) {

@@ -79,6 +79,7 @@ SIGNATURES: dict[str, tuple] = {
     "plz_linear_fwd_dense_workspace": (sz, [i64, i64, i64]),
     "plz_linear_fwd_dense_swiglu": (i32, [p, p, p, i64, i64, i64, p]),
     "plz_linear_fwd_dense_swiglu_cat": (i32, [p, p, p, p, i32, p, p, i64, i64, i64, p]),
+    "plz_linear_fwd_dense_kn": (i32, [p, p, p, p, p, sz, i64, i64, i64, p]),
     "plz_linear_bwd_x_dense": (i32, [p, p, p, p, i32, p, p, sz, i64, i64, i64, p]),
     "plz_linear_bwd_x_dense_workspace": (sz, [i64, i64, i64]),
     "plz_gumbel_philox": (i32, [p, i64, u64, u64, p]),
@@ -86,6 +87,10 @@ SIGNATURES: dict[str, tuple] = {
     "plz_gumbel_lcg_triton": (i32, [p, u32, i64, i64, p]),
     "plz_pw_ref_plan": (i64, [C.POINTER(PwRefDesc), i32, i64]),
     "plz_soft_pw_ref_batched": (i32, [p, i32, i64, i64, f32, u32, p]),
+    "plz_soft_ref_build_w": (i32, [p, i32, p, i32, i64, i32, u32, f32, i32, p, i64, i64, p]),
+    "plz_soft_ref_bwd_workspace": (sz, [i64, i64, i64]),
+    "plz_soft_ref_bwd": (i32, [p, p, p, i32, p, i32, i64, i64, i32, u32, f32, i32, p, p, p, sz,
+                               i64, i64, i64, p]),
     "plz_soft_build_w": (i32, [p, i32, p, p, f32, i32, p, p, p, i64, i64, p]),
     "plz_soft_build_w_philox": (i32, [p, i32, u64, u64, p, f32, i32, p, p, p, i64, i64, p]),
     "plz_build_w_plan": (i64, [C.POINTER(BuildWDesc), i32]),

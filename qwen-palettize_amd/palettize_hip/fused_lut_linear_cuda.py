@@ -24,7 +24,8 @@ Same names, arguments, layouts and gradient tuples as the reference
 The reference layout (one palette per 256 output channels spanning all of K) is mapped onto
 the native one (palette per output row and 256-wide K chunk) by expanding the palette; its
 gradient is summed back over the expansion. K is zero-padded to a multiple of 256 when needed
-(the padded columns multiply zeros and contribute nothing).
+(the padded columns multiply zeros and contribute nothing). The soft path with its own LCG noise
+stays in the reference layout where the sizes allow it (_soft_in_reference_layout).
 """
 from __future__ import annotations
 
@@ -295,6 +296,19 @@ def _noise_to_native(noise: Tensor, K: int, N: int, Kp: int) -> Tensor:
     return noise.contiguous()
 
 
+def _soft_in_reference_layout(x, palette, logits, N, K, group_size):
+    """True where the soft linear runs in the (K, N) order of its logits (plz_soft_ref_*): whole
+    8-element chunks along both dimensions, the palette in a type its kernels read. On
+    2560 -> 4096 at 2048 rows that takes the two plane transposes (206 us each), the noise tensor
+    and its reads out of a training pass. Other sizes go through the native layout, K padded."""
+    return (x.is_cuda and logits.is_cuda and palette.is_cuda and x.dtype == torch.bfloat16
+            and x.dim() == 2 and x.shape[0] > 0 and N > 0 and K > 0 and K % 8 == 0
+            and palette.dim() == 2 and palette.shape[1] == 4
+            and palette.shape[0] >= _groups_used(N, group_size)
+            and palette.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and all(t.data_ptr() % 16 == 0 for t in (x, logits) if t.is_contiguous()))
+
+
 def _soft_forward(ctx, x, palette, logits, bias, group_size, tau, noise, ste, semantics="cuda"):
     """Forward of fused_lut_linear_soft: W from logits + noise + palette (when ste, W_hard of
     the noisy P for "cuda" semantics or of the plain logits for "triton"; else W_soft), then
@@ -310,6 +324,24 @@ def _soft_forward(ctx, x, palette, logits, bias, group_size, tau, noise, ste, se
         raise ValueError(f"x K={x.shape[-1]} != logits K={K}")
     if N % 8:
         raise ValueError(f"N ({N}) must be a multiple of 8")
+    ctx.group_size, ctx.K, ctx.tau = group_size, K, float(tau)
+    ctx.n_groups = palette.shape[0]
+    ctx.pal_dtype, ctx.logits_dtype = palette.dtype, logits.dtype
+    ctx.has_bias = bias is not None
+    ctx.bias_dtype = None if bias is None else bias.dtype
+    ctx.ref_seed = None
+    hard = PLZ_W_HARD_PLAIN if semantics == "triton" else PLZ_W_HARD_NOISY
+    if noise is None and _soft_in_reference_layout(x, palette, logits, N, K, group_size):
+        # the reference's LCG draw, one seed per forward, in the kernels
+        seed = _next_triton_step_seed() if semantics == "triton" else _next_soft_step_seed()
+        xc, lg, pal = x.contiguous(), logits.contiguous(), palette.detach().clone()
+        w = ops.soft_ref_build_w(lg, pal, group_size, seed, float(tau),
+                                 hard if ste else PLZ_W_SOFT, semantics)
+        b = None if bias is None else bias.to(torch.bfloat16).contiguous()
+        y = ops.linear_fwd_dense_kn(xc, w, b)
+        ctx.save_for_backward(xc, pal, lg, w)
+        ctx.ref_seed, ctx.semantics = seed, semantics
+        return y
     xp = _prep_x(x, K)
     Kp = xp.shape[1]
     lg = logits_from_reference(logits, K)
@@ -322,21 +354,28 @@ def _soft_forward(ctx, x, palette, logits, bias, group_size, tau, noise, ste, se
     else:
         noise = _noise_to_native(noise, K, N, Kp)
     pal = palette_from_reference(palette, N, K, group_size)
-    hard = PLZ_W_HARD_PLAIN if semantics == "triton" else PLZ_W_HARD_NOISY
     w, _ = ops.soft_build_w(lg, noise, pal, float(tau), hard if ste else PLZ_W_SOFT)
     b = None if bias is None else bias.to(torch.bfloat16).contiguous()
     y = ops.linear_fwd_dense(xp, w, b)
     ctx.save_for_backward(xp, pal, lg, noise, w)
-    ctx.group_size, ctx.K, ctx.tau = group_size, K, float(tau)
-    ctx.n_groups = palette.shape[0]
-    ctx.pal_dtype, ctx.logits_dtype = palette.dtype, logits.dtype
-    ctx.has_bias = bias is not None
-    ctx.bias_dtype = None if bias is None else bias.dtype
     return y
 
 
 def _soft_backward(ctx, grad_y):
     """(grad_x, grad_palette, grad_logits, grad_bias) in the reference layouts."""
+    if ctx.ref_seed is not None:
+        xc, pal, lg, w = ctx.saved_tensors
+        grad_y = grad_y.contiguous()
+        need = ctx.needs_input_grad
+        grad_x = ops.linear_fwd_dense(grad_y, w) if need[0] else None  # grad_y W^T of W [K, N]
+        grad_pal = grad_logits = grad_bias = None
+        if need[1] or need[2]:
+            grad_logits, grad_pal = ops.soft_ref_bwd(xc, grad_y, lg, pal, ctx.group_size,
+                                                     ctx.ref_seed, ctx.tau, ctx.semantics,
+                                                     want_logits=need[2])
+        if ctx.has_bias and need[3]:
+            grad_bias = ops.bias_grad(grad_y).to(ctx.bias_dtype)
+        return grad_x, grad_pal if need[1] else None, grad_logits, grad_bias
     xp, pal, lg, noise, w = ctx.saved_tensors
     grad_y = grad_y.contiguous()
     grad_x = grad_pal = grad_logits = grad_bias = None

@@ -316,6 +316,22 @@ def linear_fwd_dense(x, w, bias=None, lora_t=None, lora_b=None, residual=None):
     return y
 
 
+def linear_fwd_dense_kn(x, w, bias=None):
+    """y = x w (+ bias) for a weight stored [K, N]."""
+    _need(x, "x", torch.bfloat16, 2)
+    _need(w, "w", torch.bfloat16, 2)
+    M, K = x.shape
+    N = w.shape[1]
+    if w.shape[0] != K:
+        raise ValueError("x / w shape mismatch")
+    _bias(bias, N)
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    ws = _opt_workspace(query("plz_linear_bwd_x_dense_workspace", M, K, N), x.device)
+    call("plz_linear_fwd_dense_kn", _ptr(x), _ptr(w), _ptr(bias), _ptr(y), _ptr(ws), _numel(ws), M,
+         N, K, _stream(x))
+    return y
+
+
 def linear_bwd_x_dense(grad_y, w, lora_gt=None, lora_a=None):
     _need(grad_y, "grad_y", torch.bfloat16, 2)
     _need(w, "w", torch.bfloat16, 2)
@@ -438,6 +454,55 @@ def soft_pw_reference_batched(logits_list, palette_list, group_size: int, tau: f
     call("plz_soft_pw_ref_batched", table.data_ptr(), n, int(total), group_size, float(tau),
          int(step_seed) & 0xFFFFFFFF, torch.cuda.current_stream(dev).cuda_stream)
     return outs
+
+
+def _soft_ref_shapes(logits, palette, group_size):
+    """(K, N) of reference-layout logits (4, K, N) and palette (G, 4)."""
+    if logits.dtype not in (torch.bfloat16, torch.float16):
+        raise TypeError("logits must be bf16 or fp16")
+    _need(logits, "logits", None, 3)
+    _need(palette, "palette", None, 2)
+    if palette.dtype not in _DT:
+        raise TypeError("palette must be bf16, fp16 or fp32")
+    if logits.shape[0] != 4 or palette.shape[1] != 4:
+        raise ValueError("logits (4, K, N) and palette (G, 4) expected")
+    K, N = logits.shape[1], logits.shape[2]
+    if palette.shape[0] * int(group_size) < N:
+        raise ValueError(f"palette has {palette.shape[0]} groups of {group_size} for {N} columns")
+    return K, N
+
+
+def soft_ref_build_w(logits, palette, group_size: int, seed: int, tau: float, mode: int,
+                     variant: str = "cuda"):
+    """W [K, N] bf16 of reference-layout logits (4, K, N) and palette (G, 4), the LCG noise of
+    gumbel_lcg(variant=...) drawn in the kernel: the transpose of what soft_build_w makes of the
+    native-layout tensors. K and N multiples of 8."""
+    K, N = _soft_ref_shapes(logits, palette, group_size)
+    w = torch.empty((K, N), dtype=torch.bfloat16, device=logits.device)
+    call("plz_soft_ref_build_w", _ptr(logits), _DT[logits.dtype], _ptr(palette),
+         _DT[palette.dtype], int(group_size), int(variant == "triton"), int(seed) & 0xFFFFFFFF,
+         float(tau), int(mode), _ptr(w), K, N, _stream(logits))
+    return w
+
+
+def soft_ref_bwd(x, grad_y, logits, palette, group_size: int, seed: int, tau: float,
+                 variant: str = "cuda", want_logits: bool = True):
+    """(grad_logits (4, K, N) or None, grad_palette (G, 4)) of the reference-layout soft linear, in
+    the logits' and the palette's types: soft_bwd with the noise drawn again in the kernel."""
+    K, N = _soft_ref_shapes(logits, palette, group_size)
+    _need(x, "x", torch.bfloat16, 2)
+    _need(grad_y, "grad_y", torch.bfloat16, 2)
+    M = x.shape[0]
+    if x.shape[1] != K or tuple(grad_y.shape) != (M, N):
+        raise ValueError("x / grad_y shape mismatch")
+    gl = torch.empty_like(logits) if want_logits else None
+    gp = torch.empty_like(palette)
+    ws = _workspace(query("plz_soft_ref_bwd_workspace", M, N, K), x.device)
+    call("plz_soft_ref_bwd", _ptr(x), _ptr(grad_y), _ptr(logits), _DT[logits.dtype], _ptr(palette),
+         _DT[palette.dtype], palette.shape[0], int(group_size), int(variant == "triton"),
+         int(seed) & 0xFFFFFFFF, float(tau), 0, _ptr(gl), _ptr(gp), _ptr(ws), ws.numel(), M, N, K,
+         _stream(x))
+    return gl, gp
 
 
 class PhiloxNoise:

@@ -200,3 +200,52 @@ def test_fused_compute_P_W_batched_on_student(dev):
     student.down.group_size = 128
     with pytest.raises(ValueError, match="must share group_size"):
         FL.fused_compute_P_W_batched(student, 0.5, 777)
+
+
+@pytest.mark.parametrize("semantics", ["cuda", "triton"])
+@pytest.mark.parametrize("M,K,N,GS,dt,pdt,ste,strided", [
+    (1, 8, 8, 256, torch.float16, torch.bfloat16, True, False),
+    (70, 264, 520, 100, torch.bfloat16, torch.float32, True, True),
+    (300, 512, 1032, 256, torch.float16, torch.bfloat16, False, False),
+    (2000, 1048, 264, 3, torch.float16, torch.float16, True, False),
+    (33, 256, 256, 256, torch.float16, torch.bfloat16, True, True)])
+def test_soft_reference_layout_route_against_the_native_one(dev, semantics, M, K, N, GS, dt, pdt,
+                                                            ste, strided, monkeypatch):
+    """The soft linear in (K, N) order (noise drawn in its kernels) against the same call through
+    the native layout (noise tensor, K padded): group sizes that split a lane's four columns,
+    partial groups and unused ones, strided logits, both samplers, a reduction in one and in
+    several splits. The forward weight is the same, so y differs by summation order only."""
+    g = torch.Generator().manual_seed(M + K + N)
+    logits = (torch.randn(4, K, N, generator=g) * 2).to(dt).to(dev)
+    pal = (torch.randn(-(-N // GS) + 1, 4, generator=g) * 0.02).to(pdt).to(dev)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
+    gy = torch.randn(M, N, generator=g).to(torch.bfloat16).to(dev)
+    bias = torch.randn(N, generator=g).to(torch.bfloat16).to(dev)
+    if strided:
+        logits = logits.transpose(1, 2).contiguous().transpose(1, 2)
+    outs = []
+    for native in (False, True):
+        FL._SOFT_STEP_SEED = FL._TRITON_STEP_SEED = 77
+        if native:
+            monkeypatch.setattr(FL, "_soft_in_reference_layout", lambda *a: False)
+        leaves = [t.detach().clone().requires_grad_(True) for t in (x, pal, bias)]
+        lg = logits.detach().requires_grad_(True)
+        y = FL.fused_lut_linear_soft(leaves[0], leaves[1], lg, leaves[2], GS, 0.7, ste=ste,
+                                     semantics=semantics)
+        y.backward(gy)
+        outs.append([y] + [t.grad for t in leaves] + [lg.grad])
+    for a, b, what in zip(*outs, ("y", "grad_x", "grad_palette", "grad_bias", "grad_logits")):
+        assert a.dtype == b.dtype and a.shape == b.shape, what
+        assert_close(f32(a), f32(b).astype(np.float64), what=f"{what} (routes)")
+    # the weights themselves: the hard picks bit for bit; W_soft within one bf16 ulp (2^-7
+    # relative), since the compiler may fuse the two kernels' fp32 sums differently
+    hard = ops._lib.PLZ_W_HARD_PLAIN if semantics == "triton" else PLZ_W_HARD_NOISY
+    mode = hard if ste else ops._lib.PLZ_W_SOFT
+    w = ops.soft_ref_build_w(logits.contiguous(), pal, GS, 78, 0.7, mode, semantics)
+    Kp = FL._pad_k(K)
+    noise = ops.gumbel_lcg(N, Kp, 78, device=dev, variant=semantics)
+    wn, _ = ops.soft_build_w(FL.logits_from_reference(logits, K), noise,
+                             FL.palette_from_reference(pal, N, K, GS), 0.7, mode)
+    wn = wn[:, :K].t()
+    assert torch.equal(w, wn) if ste else torch.allclose(w.float(), wn.float(), rtol=2 ** -7,
+                                                         atol=1e-8)
