@@ -151,20 +151,28 @@ class QwenLoRA(nn.Module):
         y_base = self.base(x)
         lead = x.shape[:-1]
         x_flat = x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
-        lora = _LoRAFunction.apply(x_flat, self.lora_A, self.lora_B, self.scaling)
+        if (y_base.is_cuda and y_base.dtype == torch.bfloat16 and y_base.is_contiguous()
+                and tuple(y_base.shape) == (*lead, self.lora_B.shape[0])
+                and y_base.numel() > 0 and y_base.data_ptr() % 16 == 0):
+            # the add rides in the epilogue of the t B^T GEMM, rounded as a separate add would be
+            y = _LoRAFunction.apply(x_flat, self.lora_A, self.lora_B, self.scaling,
+                                    y_base.reshape(-1, y_base.shape[-1]))
+            return y.reshape(y_base.shape)
+        lora = _LoRAFunction.apply(x_flat, self.lora_A, self.lora_B, self.scaling, None)
         return y_base + lora.reshape(*lead, -1).to(y_base.dtype)
 
 
 class _LoRAFunction(torch.autograd.Function):
-    """scale * (x A) B^T with A (in, r), B (out, r) on the skinny HIP GEMMs."""
+    """scale * (x A) B^T (+ residual [M, out]) with A (in, r), B (out, r) on the skinny HIP
+    GEMMs."""
 
     @staticmethod
-    def forward(ctx, x, A, B, scale):
+    def forward(ctx, x, A, B, scale, residual):
         from . import ops
         a_rk = A.t().contiguous()          # [r, K]
         b_nr = B.contiguous()              # [N, r]
         t = ops.lora_project(x, a_rk, scale)   # s * x A   [M, r]
-        y = ops.linear_fwd_dense(t, b_nr)      # t B^T     [M, N]
+        y = ops.linear_fwd_dense(t, b_nr, residual=residual)  # t B^T (+ residual)  [M, N]
         ctx.save_for_backward(x, a_rk, b_nr, t)
         ctx.scale = scale
         return y
@@ -177,4 +185,4 @@ class _LoRAFunction(torch.autograd.Function):
         gt = ops.lora_grad_t(gy, b_nr, ctx.scale)            # s * gy B   [M, r]
         gx = ops.linear_bwd_x_dense(gt, a_rk) if ctx.needs_input_grad[0] else None  # gt A^T
         ga, gb = ops.lora_weight_grads(x, gy, t, gt, 1.0, out_dtype=torch.bfloat16)
-        return gx, ga.t(), gb, None
+        return gx, ga.t(), gb, None, gy if ctx.needs_input_grad[4] else None
