@@ -171,7 +171,7 @@ def lib():
 
 def call(name: str, *args) -> int:
     """Calls an int-returning entry point and raises PalettizeError on failure."""
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != PLZ_OK:
         msg = lib().plz_last_error().decode(errors="replace")
         raise PalettizeError(f"{name} failed (status {rc}): {msg}")
@@ -179,4 +179,4 @@ def call(name: str, *args) -> int:
 
 
 def query(name: str, *args) -> int:
-    return int(getattr(lib(), name)(*args))
+    return int(getattr(_lib or lib(), name)(*args))

@@ -23,7 +23,8 @@ _DT = {torch.bfloat16: _lib.PLZ_DT_BF16, torch.float16: _lib.PLZ_DT_FP16,
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the raw handle, without a Stream object (2 us less per call)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _on_gpu(t: torch.Tensor) -> bool:
@@ -31,6 +32,9 @@ def _on_gpu(t: torch.Tensor) -> bool:
 
 
 def _need(t: torch.Tensor, name: str, dtype=None, ndim=None) -> torch.Tensor:
+    if (isinstance(t, torch.Tensor) and t.is_cuda and (dtype is None or t.dtype == dtype)
+            and (ndim is None or t.dim() == ndim) and t.is_contiguous()):
+        return t
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a tensor")
     if not _on_gpu(t):
@@ -872,7 +876,7 @@ class GemvGroup:
         self.n = len(items)
 
     def run(self):
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = torch._C._cuda_getCurrentRawStream(self.device.index)
         if self.layout == _lib.PLZ_GEMV_PLANES:
             call("plz_lut_gemv_grouped_planes", self.table.data_ptr(), self.n, self.total_blocks,
                  self.M, self.max_K, _ptr(self.workspace), _numel(self.workspace), stream)
