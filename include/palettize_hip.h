@@ -621,6 +621,14 @@ int plz_head_norm_rope_bwd(const uint16_t* x, const uint16_t* weight, const floa
                            const float* cos_table, const float* sin_table, const uint16_t* grad_y,
                            uint16_t* grad_x, int64_t rows, int64_t seq, int heads, int head_dim,
                            void* stream);
+/* Reference palettes (G, 4) (bf16 / fp16 / fp32, row n in group n / group_size) to the native fp32
+ * [N, kg, 4], and a native palette gradient summed back over a group's rows and kg (groups
+ * without rows: zero), in a fixed order in fp32. */
+int plz_palette_expand(const void* palette, int dtype, float* out, int64_t N, int64_t kg,
+                       int64_t group_size, void* stream);
+int plz_palette_fold(const float* grad, void* out, int dtype, int64_t n_groups, int64_t N,
+                     int64_t kg, int64_t group_size, void* stream);
+
 /* Causal grouped-query attention forward (flash-style): q, o bf16 [batch, seq, heads, 128],
  * k, v bf16 [batch, seq, kv_heads, 128], heads % kv_heads == 0, seq % 128 == 0;
  * o = softmax(q k^T * scale, causal) v per head (kv head = head / (heads / kv_heads)),

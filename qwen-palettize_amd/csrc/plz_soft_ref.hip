@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256) void bwd_kernel(const Weights w, const float* 
   }
 }
 
-// grad_palette (G, 4): group g = its columns' sums over all row blocks, fixed order; groups that
+// Palette gradient (G, 4): group g = its columns' sums over all row blocks, fixed order; groups that
 // no column uses are zero. One workgroup per group.
 __global__ __launch_bounds__(512) void pal_kernel(const float4* __restrict__ cols, int64_t blocks,
                                                   int64_t N, int64_t group_size, void* out,
@@ -231,12 +231,20 @@ __global__ __launch_bounds__(512) void pal_kernel(const float4* __restrict__ col
   const int64_t g = blockIdx.x, n0 = g * group_size;
   const int64_t nc = n0 >= N ? 0 : (n0 + group_size < N ? group_size : N - n0);
   float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int64_t c = threadIdx.x & 255; c < nc; c += 256) {  // two row blocks of 256 columns a step
-    const float4* p = cols + n0 + c;
+  if (blocks == 1) {
 #pragma unroll 8
-    for (int64_t b = threadIdx.x >> 8; b < blocks; b += 2) {
-      const float4 d = p[b * N];
+    for (int64_t c = threadIdx.x; c < nc; c += 512) {
+      const float4 d = cols[n0 + c];
       s.x += d.x; s.y += d.y; s.z += d.z; s.w += d.w;
+    }
+  } else {
+    for (int64_t c = threadIdx.x & 255; c < nc; c += 256) {  // two row blocks of 256 columns a step
+      const float4* p = cols + n0 + c;
+#pragma unroll 8
+      for (int64_t b = threadIdx.x >> 8; b < blocks; b += 2) {
+        const float4 d = p[b * N];
+        s.x += d.x; s.y += d.y; s.z += d.z; s.w += d.w;
+      }
     }
   }
   red[threadIdx.x] = s;
@@ -250,6 +258,16 @@ __global__ __launch_bounds__(512) void pal_kernel(const float4* __restrict__ col
   __syncthreads();
   if (threadIdx.x < 4)
     store_elem(out, dtype, 4 * g + threadIdx.x, reinterpret_cast<const float*>(red)[threadIdx.x]);
+}
+
+// One thread per native palette entry: a 16-byte store of its row's group.
+__global__ void expand_kernel(const void* pal, int dtype, float4* __restrict__ out, int64_t total,
+                              int64_t kg, int64_t group_size) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= total) return;
+  const int64_t g = t / kg / group_size * 4;
+  out[t] = make_float4(elem(pal, dtype, g), elem(pal, dtype, g + 1), elem(pal, dtype, g + 2),
+                       elem(pal, dtype, g + 3));
 }
 
 static int64_t row_blocks(int64_t K) { return (K + KR - 1) / KR; }
@@ -279,6 +297,37 @@ using namespace plz;
 using namespace plz::sref;
 
 extern "C" {
+
+int plz_palette_expand(const void* palette, int dtype, float* out, int64_t N, int64_t kg,
+                       int64_t group_size, void* stream) {
+  PLZ_REQUIRE(N >= 0 && kg >= 0 && group_size > 0, "plz_palette_expand: bad shape");
+  PLZ_REQUIRE(dtype == PLZ_DT_BF16 || dtype == PLZ_DT_FP16 || dtype == PLZ_DT_FP32,
+              "plz_palette_expand: palette must be bf16, fp16 or fp32");
+  if (N == 0 || kg == 0) return PLZ_OK;
+  PLZ_REQUIRE(palette && out && ((uintptr_t)out & 15) == 0,
+              "plz_palette_expand: null or misaligned pointer");
+  const int64_t total = N * kg;
+  hipLaunchKernelGGL(expand_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream, palette, dtype, reinterpret_cast<float4*>(out), total, kg,
+                     group_size);
+  return check_launch("plz_palette_expand");
+}
+
+int plz_palette_fold(const float* grad, void* out, int dtype, int64_t n_groups, int64_t N,
+                     int64_t kg, int64_t group_size, void* stream) {
+  PLZ_REQUIRE(N > 0 && kg > 0 && group_size > 0 && n_groups <= 0x7fffffff &&
+                  n_groups >= (N + group_size - 1) / group_size,
+              "plz_palette_fold: bad shape");
+  PLZ_REQUIRE(dtype == PLZ_DT_BF16 || dtype == PLZ_DT_FP16 || dtype == PLZ_DT_FP32,
+              "plz_palette_fold: out must be bf16, fp16 or fp32");
+  PLZ_REQUIRE(grad && out && ((uintptr_t)grad & 15) == 0,
+              "plz_palette_fold: null or misaligned pointer");
+  // [N, kg, 4] as one block of N kg columns in groups of group_size kg
+  hipLaunchKernelGGL(pal_kernel, dim3((unsigned)n_groups), dim3(512), 0, (hipStream_t)stream,
+                     reinterpret_cast<const float4*>(grad), (int64_t)1, N * kg, group_size * kg,
+                     out, dtype);
+  return check_launch("plz_palette_fold");
+}
 
 int plz_soft_ref_build_w(const uint16_t* logits, int logits_dtype, const void* palette,
                          int palette_dtype, int64_t group_size, int triton_hash, uint32_t seed,

@@ -52,6 +52,8 @@ SIGNATURES: dict[str, tuple] = {
     "plz_pack_indices": (i32, [p, p, i64, i64, p]),
     "plz_unpack_indices": (i32, [p, p, i64, i64, p]),
     "plz_dequant": (i32, [p, p, p, i64, i64, p]),
+    "plz_palette_expand": (i32, [p, i32, p, i64, i64, i64, p]),
+    "plz_palette_fold": (i32, [p, p, i32, i64, i64, i64, i64, p]),
     "plz_attn_fwd": (i32, [p, p, p, p, p, i32, i32, i32, i32, i32, f32, p]),
     "plz_attn_bwd_workspace": (sz, [i32, i32, i32]),
     "plz_attn_bwd": (i32, [p, p, p, p, p, p, p, p, p, p, sz, i32, i32, i32, i32, i32, f32, p]),

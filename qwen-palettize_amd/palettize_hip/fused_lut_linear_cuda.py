@@ -111,23 +111,28 @@ def palette_from_reference(palette: Tensor, N: int, K: int, group_size: int) -> 
         raise ValueError(f"G mismatch: {N} rows in groups of {group_size} need {need} palettes, "
                          f"palette has {G}")
     kg = _pad_k(K) // 256
+    if palette.is_cuda and palette.dtype in ops._DT and N > 0 and kg > 0:
+        return ops.palette_expand(palette.detach().contiguous(), N, kg, group_size)
     per_row = palette[:need].float().repeat_interleave(group_size, dim=0)[:N]  # [N, 4]
     return per_row[:, None, :].expand(N, kg, 4).contiguous()
 
 
-def palette_grad_to_reference(grad: Tensor, group_size: int, n_groups: int | None = None) -> Tensor:
-    """native [N, KG, 4] -> reference (G, 4): sum over the rows of a group and over KG; groups
-    no row uses (G above ceil(N / group_size)) get zero."""
+def palette_grad_to_reference(grad: Tensor, group_size: int, n_groups: int | None = None,
+                              dtype: torch.dtype = torch.float32) -> Tensor:
+    """native [N, KG, 4] -> reference (G, 4) in ``dtype``: sum over the rows of a group and over
+    KG; groups no row uses (G above ceil(N / group_size)) get zero."""
     N = grad.shape[0]
     need = _groups_used(N, group_size)
     G = need if n_groups is None else int(n_groups)
+    if grad.is_cuda and dtype in ops._DT and grad.numel() > 0:
+        return ops.palette_fold(grad, G, group_size, dtype)
     per_row = grad.sum(dim=1)  # [N, 4]
     if need * group_size != N:
         per_row = F.pad(per_row, (0, 0, 0, need * group_size - N))
     out = per_row.view(need, group_size, 4).sum(dim=1)
     if G > need:
         out = F.pad(out, (0, 0, 0, G - need))
-    return out
+    return out.to(dtype)
 
 
 def _prep_x(x: Tensor, K: int) -> Tensor:
@@ -172,7 +177,7 @@ class CUDAFusedLUTLinear(torch.autograd.Function):
             grad_x = ops.lut_linear_bwd_x(grad_y, packed, pal)[:, : ctx.K].contiguous()
         if ctx.needs_input_grad[1]:
             g = ops.lut_linear_bwd_palette(xp, grad_y, packed)
-            grad_pal = palette_grad_to_reference(g, ctx.group_size, ctx.n_groups).to(ctx.pal_dtype)
+            grad_pal = palette_grad_to_reference(g, ctx.group_size, ctx.n_groups, ctx.pal_dtype)
         if ctx.bias_requires_grad:
             grad_bias = ops.bias_grad(grad_y).to(ctx.bias_dtype)
         return grad_x, grad_pal, None, grad_bias, None
@@ -232,7 +237,7 @@ class PreTransposedLUTLinear(torch.autograd.Function):
             grad_x = ops.lut_linear_fwd(gyp, packed, pal)
         if ctx.needs_input_grad[1]:
             g = ops.lut_linear_bwd_palette(gyp, xc, packed)      # [in, Kp'/256, 4]
-            grad_pal = palette_grad_to_reference(g, ctx.group_size, ctx.n_groups).to(ctx.pal_dtype)
+            grad_pal = palette_grad_to_reference(g, ctx.group_size, ctx.n_groups, ctx.pal_dtype)
         if ctx.bias_requires_grad:
             grad_bias = ops.bias_grad(gy).to(ctx.bias_dtype)
         return grad_x, grad_pal, None, grad_bias, None
@@ -386,7 +391,8 @@ def _soft_backward(ctx, grad_y):
         if ctx.needs_input_grad[2]:
             grad_logits = gl[:, : ctx.K, :].permute(2, 1, 0).contiguous().to(ctx.logits_dtype)
         if ctx.needs_input_grad[1]:
-            grad_pal = palette_grad_to_reference(gp, ctx.group_size, ctx.n_groups).to(ctx.pal_dtype)
+            grad_pal = palette_grad_to_reference(gp, ctx.group_size, ctx.n_groups,
+                                                 ctx.pal_dtype)
     if ctx.has_bias and ctx.needs_input_grad[3]:
         grad_bias = ops.bias_grad(grad_y).to(ctx.bias_dtype)
     return grad_x, grad_pal, grad_logits, grad_bias

@@ -109,6 +109,33 @@ def dequant(packed: torch.Tensor, palette: torch.Tensor) -> torch.Tensor:
     return w
 
 
+# ---- reference-layout palettes ----------------------------------------------------------
+def palette_expand(palette, N: int, kg: int, group_size: int):
+    """(G, 4) palette -> native fp32 [N, kg, 4], row n from group n // group_size."""
+    _need(palette, "palette", None, 2)
+    if palette.dtype not in _DT or palette.shape[1] != 4:
+        raise TypeError("palette must be (G, 4) bf16, fp16 or fp32")
+    if palette.shape[0] * int(group_size) < N:
+        raise ValueError(f"palette has {palette.shape[0]} groups of {group_size} for {N} rows")
+    out = torch.empty((N, kg, 4), dtype=torch.float32, device=palette.device)
+    call("plz_palette_expand", _ptr(palette), _DT[palette.dtype], _ptr(out), N, kg,
+         int(group_size), _stream(palette))
+    return out
+
+
+def palette_fold(grad, n_groups: int, group_size: int, dtype=torch.float32):
+    """native fp32 [N, kg, 4] -> (n_groups, 4): the sum over a group's rows and over kg, in fp32;
+    groups without rows are zero."""
+    _need(grad, "grad", torch.float32, 3)
+    N, kg = grad.shape[0], grad.shape[1]
+    if n_groups * int(group_size) < N:
+        raise ValueError(f"{n_groups} groups of {group_size} for {N} rows")
+    out = torch.empty((n_groups, 4), dtype=dtype, device=grad.device)
+    call("plz_palette_fold", _ptr(grad), _ptr(out), _DT[dtype], int(n_groups), N, kg,
+         int(group_size), _stream(grad))
+    return out
+
+
 # ---- hard linear --------------------------------------------------------------------
 def _lora_pair(a, b, first: str, second: str, rows_a: int, rows_b: int):
     if (a is None) != (b is None):

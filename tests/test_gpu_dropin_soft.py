@@ -249,3 +249,25 @@ def test_soft_reference_layout_route_against_the_native_one(dev, semantics, M, K
     wn = wn[:, :K].t()
     assert torch.equal(w, wn) if ste else torch.allclose(w.float(), wn.float(), rtol=2 ** -7,
                                                          atol=1e-8)
+
+
+@pytest.mark.parametrize("N,kg,GS,G", [(8, 1, 256, 1), (1032, 3, 100, 11), (4096, 10, 256, 16),
+                                       (264, 38, 3, 90)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+def test_palette_expand_and_fold(dev, N, kg, GS, G, dt):
+    """Reference palettes to the native layout and the gradient back: partial, many and unused
+    groups. The expansion is exact; a group's sum is fp32 in another order (n terms of random
+    sign: error below n 2^-24 of the sum of magnitudes), rounded to the palette's type."""
+    g = torch.Generator().manual_seed(N + kg)
+    pal = torch.randn(G, 4, generator=g).to(dt).to(dev)
+    want = pal.float().repeat_interleave(GS, 0)[:N][:, None].expand(N, kg, 4)
+    assert torch.equal(FL.palette_from_reference(pal, N, 256 * kg, GS), want)
+    grad = torch.randn(N, kg, 4, generator=g).to(dev)
+    got = FL.palette_grad_to_reference(grad, GS, G, dt)
+    ref, mag = (torch.zeros(G, 4, dtype=torch.float64, device=dev) for _ in range(2))
+    rows = torch.arange(N, device=dev) // GS
+    ref.index_add_(0, rows, grad.double().sum(1))
+    mag.index_add_(0, rows, grad.double().abs().sum(1))
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dt]
+    assert got.dtype == dt and bool(((got.double() - ref).abs() <=
+                                     eps * ref.abs() + GS * kg * 2.0 ** -24 * mag + 1e-7).all())
