@@ -180,8 +180,25 @@ int plz_linear_fwd_dense_swiglu(const uint16_t* x, const uint16_t* w_gate_up, ui
 int plz_linear_fwd_dense_swiglu_cat(const uint16_t* x, const uint16_t* w, const uint16_t* lora_t,
                                     const uint16_t* lora_b, int rank, uint16_t* y, uint16_t* h,
                                     int64_t M, int64_t F, int64_t K, void* stream);
-/* y = x w (+ bias) for a weight stored [K, N]; the workspace is
- * plz_linear_bwd_x_dense_workspace(M, K, N). */
+/* How a LUT GEMM of rows x outputs over a reduction (forward M, N, K; grad_x M, K, N) is fastest:
+ * 0 in one pass (plz_lut_linear_fwd / _bwd_x); 1 plz_dequant and a tiled GEMM below on the bf16 W;
+ * 2 so too, which those entries do themselves in the workspace that their queries ask for. */
+int plz_lut_linear_staged(int64_t rows, int64_t outputs, int64_t reduction);
+/* plz_linear_fwd_dense (with an optional residual) and plz_linear_bwd_x_dense on the GEMM core,
+ * 128x128 or 256x256 tiles, that is the faster one for the shape. Where that is the smaller one,
+ * the fp32 sums over K (N) are split differently from the dense entries'. The workspace (optional:
+ * without it nothing is split) is plz_linear_tiled_workspace(M, N, K) for the forward and
+ * plz_linear_tiled_workspace(M, K, N) for grad_x. */
+size_t plz_linear_tiled_workspace(int64_t M, int64_t N, int64_t K);
+int plz_linear_fwd_tiled(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                         const uint16_t* lora_t, const uint16_t* lora_b, int rank,
+                         const uint16_t* residual, uint16_t* y, void* workspace,
+                         size_t workspace_bytes, int64_t M, int64_t N, int64_t K, void* stream);
+int plz_linear_bwd_x_tiled(const uint16_t* grad_y, const uint16_t* w, const uint16_t* lora_gt,
+                           const uint16_t* lora_a, int rank, uint16_t* grad_x, void* workspace,
+                           size_t workspace_bytes, int64_t M, int64_t N, int64_t K, void* stream);
+/* y = x w (+ bias) for a weight stored [K, N], on either core; the workspace is
+ * plz_linear_tiled_workspace(M, N, K). */
 int plz_linear_fwd_dense_kn(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y,
                             void* workspace, size_t workspace_bytes, int64_t M, int64_t N,
                             int64_t K, void* stream);

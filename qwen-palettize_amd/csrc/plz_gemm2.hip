@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "plz_gemm2.cuh"
+#include "plz_mid.h"
 #include "plz_skinny.h"
 #include "plz_soft_ref.h"
 #include "palettize_hip.h"
@@ -720,31 +721,6 @@ __device__ __forceinline__ void stage_tile_bf16(const Args& g, const f32x16 (&ac
       }
   __syncthreads();
 }
-// 8 stored bf16 values plus 8 bf16 residual values, each sum rounded to bf16: what a bf16 tensor
-// add of the residual to the GEMM's bf16 output computes
-__device__ __forceinline__ u32x4 add_residual8(u32x4 v, const uint16_t* r) {
-  const uint4 q = *reinterpret_cast<const uint4*>(r);
-  const uint32_t rs[4] = {q.x, q.y, q.z, q.w};
-  u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    o[e] = f2bf2(bf2f(v[e] & 0xffffu) + bf2f(rs[e] & 0xffffu), bf2f(v[e] >> 16) + bf2f(rs[e] >> 16));
-  return o;
-}
-
-// 8 stored bf16 values of grad_h at (i, j) through the SwiGLU backward (g.sw_pre set): its gate
-// and up gradients go to columns j and J + j of the [I, 2J] output
-__device__ __forceinline__ void store_swiglu_bwd8(const Args& g, u32x4 v, uint16_t* C, int64_t i,
-                                                  int64_t j) {
-  const uint16_t* pre = g.sw_pre + i * g.ld_sw + j;
-  uint4 gg, gu;
-  swiglu_bwd8(*reinterpret_cast<const uint4*>(pre), *reinterpret_cast<const uint4*>(pre + g.J),
-              make_uint4(v[0], v[1], v[2], v[3]), gg, gu);
-  const u32x4 a = {gg.x, gg.y, gg.z, gg.w}, b = {gu.x, gu.y, gu.z, gu.w};
-  __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(C + i * g.ldc + j));
-  __builtin_nontemporal_store(b, reinterpret_cast<u32x4*>(C + i * g.ldc + g.J + j));
-}
-
 __device__ __forceinline__ void store_tile_bf16(const Args& g, const f32x16 (&acc)[WT_I][WT_J],
                                                 lds_u8* st, int64_t i0, int64_t j0, int wi,
                                                 int wj, int lane) {
@@ -761,7 +737,7 @@ __device__ __forceinline__ void store_tile_bf16(const Args& g, const f32x16 (&ac
       // streaming store: the output is not read again by this launch, so it should not take
       // cache lines from the operands the other workgroups are still reading
       if (g.sw_pre)
-        store_swiglu_bwd8(g, v, C, i, j);
+        store_swiglu_bwd8(v, g.sw_pre, g.ld_sw, C, g.ldc, g.J, i, j);
       else
         __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(C + i * g.ldc + j));
     }
@@ -1389,7 +1365,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void tail_reduce_kernel(const Args g)
       u32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(st + row * EPI_RS + c8 * 2);
       if (g.res) v = add_residual8(v, g.res + i * g.ldres + j);
       if (g.sw_pre)
-        store_swiglu_bwd8(g, v, C, i, j);
+        store_swiglu_bwd8(v, g.sw_pre, g.ld_sw, C, g.ldc, g.J, i, j);
       else
         __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(C + i * g.ldc + j));
     }
@@ -1677,12 +1653,64 @@ static size_t soft_pal_bytes(int64_t N, int64_t K) { return (size_t)N * (K / 128
 using namespace plz;
 using namespace plz::g2;
 
+// Modelled time (us) of the 256x256 core on C CUs: whole waves at `per` us a stage, then the last
+// wave as tail_plan splits it (512 KB of partials a part at 5 TB/s and the reduce launch). Per
+// stage 1.4 dense, 1.55 with the LUT operand (777 x 9728 x 2560: 58.5 and 67 us).
+static double core256_us(int64_t I, int64_t J, int64_t R, double per) {
+  const int64_t tiles = ((I + TILE - 1) / TILE) * ((J + TILE - 1) / TILE), C = cu_count();
+  const double st = (double)((R + BK - 1) / BK);
+  double t = (double)(tiles / C) * (st * per + 6.0);
+  const int64_t rem = tiles % C;
+  if (rem > 0) {
+    const TailPlan p = tail_plan(I, J, R);
+    t += p.split < 2 ? st * per + 6.0
+                     : (double)(p.len / BK) * per + 13.0 +
+                           (double)rem * p.split * 2.0 * TILE * TILE * 4 / 5.0e6;
+  }
+  return t;
+}
+constexpr int64_t kMidMaxElems = (int64_t)1 << 31;
+// Dense GEMM of I x J outputs: the 128x128 core where its model is the faster one (z its splits),
+// else z = 0. us (optional): the chosen core's modelled time.
+static int dense_splits(int64_t I, int64_t J, int64_t R, double* us = nullptr) {
+  const double big = core256_us(I, J, R, 1.4);
+  if (I * R >= kMidMaxElems || J * R >= kMidMaxElems) {  // the 128x128 core's 32-bit offsets
+    if (us) *us = big;
+    return 0;
+  }
+  const mid::Plan p = mid::plan(I, J, R, cu_count());
+  const bool m = p.us < 0.95 * big;
+  if (us) *us = m ? p.us : big;
+  return m ? p.z : 0;
+}
+// ... with the workspace at hand: unsplit where it does not hold the splits' partials
+static bool mid_splits(int64_t I, int64_t J, int64_t R, void* workspace, size_t workspace_bytes,
+                       int& z) {
+  z = dense_splits(I, J, R);
+  if (z > 1 && (!workspace || !a16(workspace) || workspace_bytes < mid::workspace(I, J, z))) z = 1;
+  return z > 0;
+}
+// Workspace of a dense GEMM on the core chosen for its shape.
+static size_t dense_bytes(int64_t I, int64_t J, int64_t R) {
+  const int z = dense_splits(I, J, R);
+  return z > 0 ? mid::workspace(I, J, z) : tail_bytes(I, J, R);
+}
+
 // From this many rows the forward and grad_x dequantise W into the workspace and run the
 // dense GEMM on it: the LUT GEMMs rebuild each W tile once per 256-row tile of the activations
 // (the forward in registers, grad_x in LDS; 10-25% of their time), while dequantising once
 // costs N*K*(0.25 + 2) bytes written and read back, which a 4096-row GEMM hides several times
 // over.
 constexpr int64_t kStagedRows = 4096;
+// With fewer rows dequantising pays (2.9 us + 0.385 us per million weights) where the dense GEMM
+// then runs on the 128x128 core and the models say so. In us, LUT -> dequantise + dense: forward
+// 2560 -> 4096 at M = 128 / 1000 37 -> 26 / 53 -> 39, 9728 -> 2560 at M = 128 65 -> 36;
+// 777 x 2560 -> 9728 stays (67 against 71). The skinny forward's rows stay with it.
+static bool staged_rows(int64_t I, int64_t J, int64_t R) {
+  double us;
+  return I > sk::kMaxRows && dense_splits(I, J, R, &us) > 0 &&
+         us + 2.9 + 0.385e-6 * (double)J * (double)R < 0.97 * core256_us(I, J, R, 1.55);
+}
 // Tile-rows walked together by the dense GEMMs (consecutive workgroups share an x / grad_y
 // panel within groups of this many tile-rows). Measured on the hard step at M = 16384: 4 (and
 // 2, 6) 1085-1092 TFLOP/s against 1081 for 8, 1067-1069 for 16, 1053 for a column walk.
@@ -1945,11 +1973,20 @@ size_t plz_linear_fwd_dense_workspace(int64_t M, int64_t N, int64_t K) {
   return M > 0 && N > 0 && K > 0 ? tail_bytes(M, N, K) : 0;
 }
 
+int plz_lut_linear_staged(int64_t I, int64_t J, int64_t R) {
+  if (I <= 0 || J <= 0 || R <= 0) return 0;
+  return I >= kStagedRows ? 2 : staged_rows(I, J, R) ? 1 : 0;
+}
+
+size_t plz_linear_tiled_workspace(int64_t M, int64_t N, int64_t K) {
+  return M > 0 && N > 0 && K > 0 ? dense_bytes(M, N, K) : 0;
+}
+
 static int linear_fwd_dense(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
                             const uint16_t* lora_t, const uint16_t* lora_b, int rank,
                             const uint16_t* residual, uint16_t* y, void* workspace,
                             size_t workspace_bytes, int64_t M, int64_t N, int64_t K, void* stream,
-                            const char* what) {
+                            const char* what, bool tiled = false) {
   PLZ_REQUIRE(M >= 0 && N >= 0 && K >= 0, "%s: negative shape", what);
   PLZ_REQUIRE(K % 8 == 0 && N % 8 == 0, "%s: K and N must be multiples of 8", what);
   PLZ_REQUIRE(rank >= 0 && rank <= BK && rank % 8 == 0,
@@ -1959,6 +1996,11 @@ static int linear_fwd_dense(const uint16_t* x, const uint16_t* w, const uint16_t
               "%s: x, w, y must be non-null; x, w 16-byte aligned", what);
   PLZ_REQUIRE(rank == 0 || (lora_t && lora_b && a16(lora_t) && a16(lora_b)),
               "%s: rank > 0 needs 16-byte aligned lora_t and lora_b", what);
+  int z;
+  if (tiled && mid_splits(M, N, K, workspace, workspace_bytes, z)) {
+    mid::Args m = {x, K, w, K, M, N, K, lora_t, lora_b, rank, y, N, bias, residual, N};
+    return mid::launch(m, false, z, cu_count(), workspace, (hipStream_t)stream, what);
+  }
   Args g = {};
   g.a = x; g.lda = K; g.b = w; g.ldb = K;
   g.I = M; g.J = N; g.R = K;
@@ -1977,6 +2019,16 @@ int plz_linear_fwd_dense(const uint16_t* x, const uint16_t* w, const uint16_t* b
                          void* stream) {
   return linear_fwd_dense(x, w, bias, lora_t, lora_b, rank, nullptr, y, workspace,
                           workspace_bytes, M, N, K, stream, "plz_linear_fwd_dense");
+}
+
+int plz_linear_fwd_tiled(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                         const uint16_t* lora_t, const uint16_t* lora_b, int rank,
+                         const uint16_t* residual, uint16_t* y, void* workspace,
+                         size_t workspace_bytes, int64_t M, int64_t N, int64_t K, void* stream) {
+  PLZ_REQUIRE(M == 0 || N == 0 || !residual || (a16(residual) && y && a16(y)),
+              "plz_linear_fwd_tiled: residual and y must be 16-byte aligned");
+  return linear_fwd_dense(x, w, bias, lora_t, lora_b, rank, residual, y, workspace,
+                          workspace_bytes, M, N, K, stream, "plz_linear_fwd_tiled", true);
 }
 
 int plz_linear_fwd_dense_residual(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
@@ -2037,7 +2089,8 @@ size_t plz_linear_bwd_x_dense_workspace(int64_t M, int64_t N, int64_t K) {
 static int linear_bwd_x_dense(const uint16_t* grad_y, const uint16_t* w, const uint16_t* lora_gt,
                               const uint16_t* lora_a, int rank, const uint16_t* sw_pre,
                               const uint16_t* bias, uint16_t* grad_x, void* workspace, size_t workspace_bytes, int64_t M,
-                              int64_t N, int64_t K, void* stream, const char* what) {
+                              int64_t N, int64_t K, void* stream, const char* what,
+                              bool tiled = false) {
   PLZ_REQUIRE(M >= 0 && N >= 0 && K >= 0, "%s: negative shape", what);
   PLZ_REQUIRE(K % 8 == 0 && N % 8 == 0, "%s: K and N must be multiples of 8", what);
   PLZ_REQUIRE(rank >= 0 && rank <= BK && rank % 8 == 0,
@@ -2047,6 +2100,12 @@ static int linear_bwd_x_dense(const uint16_t* grad_y, const uint16_t* w, const u
               "%s: grad_y, w, grad_x must be non-null; grad_y, w aligned", what);
   PLZ_REQUIRE(rank == 0 || (lora_gt && lora_a && a16(lora_gt) && a16(lora_a)),
               "%s: rank > 0 needs 16-byte aligned lora_gt and lora_a", what);
+  int z;
+  if (tiled && mid_splits(M, K, N, workspace, workspace_bytes, z)) {
+    mid::Args m = {grad_y, N, w, K, M, K, N, lora_gt, lora_a, rank, grad_x, K, bias,
+                   nullptr, 0};
+    return mid::launch(m, true, z, cu_count(), workspace, (hipStream_t)stream, what);
+  }
   Args g = {};
   g.a = grad_y; g.lda = N;
   g.b = w; g.ldb = K;  // B(j=k, r=n) = w[n, k]   (Col tile)
@@ -2069,11 +2128,19 @@ int plz_linear_bwd_x_dense(const uint16_t* grad_y, const uint16_t* w, const uint
                             workspace_bytes, M, N, K, stream, "plz_linear_bwd_x_dense");
 }
 
+int plz_linear_bwd_x_tiled(const uint16_t* grad_y, const uint16_t* w, const uint16_t* lora_gt,
+                           const uint16_t* lora_a, int rank, uint16_t* grad_x, void* workspace,
+                           size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
+                           void* stream) {
+  return linear_bwd_x_dense(grad_y, w, lora_gt, lora_a, rank, nullptr, nullptr, grad_x, workspace,
+                            workspace_bytes, M, N, K, stream, "plz_linear_bwd_x_tiled", true);
+}
+
 int plz_linear_fwd_dense_kn(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y,
                             void* workspace, size_t workspace_bytes, int64_t M, int64_t N,
                             int64_t K, void* stream) {
   return linear_bwd_x_dense(x, w, nullptr, nullptr, 0, nullptr, bias, y, workspace,
-                            workspace_bytes, M, K, N, stream, "plz_linear_fwd_dense_kn");
+                            workspace_bytes, M, K, N, stream, "plz_linear_fwd_dense_kn", true);
 }
 
 int plz_linear_bwd_x_dense_swiglu(const uint16_t* grad_y, const uint16_t* w,

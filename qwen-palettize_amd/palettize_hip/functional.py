@@ -26,10 +26,10 @@ def _c(t):
 
 
 class LUTLinearFunction(torch.autograd.Function):
-    """Where the library dequantises W for the forward GEMM (from 4096 rows, see
-    ops.lut_linear_staged) and x needs a gradient, the bf16 W is kept for the backward's
-    grad_x instead of being dequantised a second time (N*K*2 bytes held from forward to
-    backward); without a gradient for x nothing reads it, and it is dropped after the GEMM."""
+    """Where the forward dequantises W and runs a dense GEMM on it (ops.lut_linear_staged) and x
+    needs a gradient, the bf16 W is kept for the backward's grad_x instead of being dequantised a
+    second time (N*K*2 bytes held from forward to backward); without a gradient for x nothing
+    reads it, and it is dropped after the GEMM."""
 
     @staticmethod
     def forward(ctx, x, packed, palette, bias, lora_a, lora_b, lora_scale):
@@ -39,7 +39,7 @@ class LUTLinearFunction(torch.autograd.Function):
         w = None
         if ops.lut_linear_staged(x.shape[0], packed.shape[0], x.shape[1]):
             w = ops.dequant(packed, palette)
-            y = ops.linear_fwd_dense(x, w, bias, t, lora_b)
+            y = ops.linear_fwd_dense(x, w, bias, t, lora_b, tiled=True)
             if not ctx.needs_input_grad[0]:
                 w = None
         else:
@@ -66,7 +66,7 @@ class LUTLinearFunction(torch.autograd.Function):
             gt = ops.lora_grad_t(gy, lora_b, ctx.lora_scale)
         grad_x = None
         if need_x:
-            grad_x = (ops.linear_bwd_x_dense(gy, w, gt, lora_a) if w is not None else
+            grad_x = (ops.linear_bwd_x_dense(gy, w, gt, lora_a, tiled=True) if w is not None else
                       ops.lut_linear_bwd_x(gy, packed, palette, gt, lora_a))
         grad_bias = ops.bias_grad(gy).to(ctx.bias_dtype) if (ctx.has_bias and need_b) else None
         grad_pal = grad_a = grad_b = None
@@ -121,8 +121,12 @@ class SoftLUTLinearFunction(torch.autograd.Function):
             ctx.grad_sq = prebuilt[2] if len(prebuilt) > 2 else None
             ctx.probs = prebuilt[3] if len(prebuilt) > 3 else None
         t = ops.lora_project(x, lora_a, lora_scale) if lora_a is not None else None
+        # a training step that builds its weights itself (prebuilt) keeps one order of sums at every
+        # batch size; a standalone linear takes the faster GEMM core
+        ctx.tiled = prebuilt is None
         y = ops.linear_fwd_dense(x, w, bias, t, lora_b,
-                                 residual=None if residual is None else residual.contiguous())
+                                 residual=None if residual is None else residual.contiguous(),
+                                 tiled=ctx.tiled)
         # a Philox noise descriptor is redrawn in the backward's epilogue, not stored; with the
         # forward's P kept, no noise is needed at all
         ctx.philox = noise if isinstance(noise, ops.PhiloxNoise) else None
@@ -165,7 +169,8 @@ class SoftLUTLinearFunction(torch.autograd.Function):
             grad_x = torch.empty(1, dtype=gy.dtype, device=gy.device).expand(x.shape)
             link.marker = grad_x.data_ptr()
         else:
-            grad_x = ops.linear_bwd_x_dense(gy, w, gt, lora_a) if need_x else None
+            grad_x = (ops.linear_bwd_x_dense(gy, w, gt, lora_a, tiled=ctx.tiled) if need_x
+                      else None)
         grad_logits = grad_pal = grad_a = grad_b = None
         if fused:
             sq = ctx.grad_sq if need_log else None

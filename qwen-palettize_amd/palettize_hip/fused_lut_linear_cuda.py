@@ -372,7 +372,8 @@ def _soft_backward(ctx, grad_y):
         xc, pal, lg, w = ctx.saved_tensors
         grad_y = grad_y.contiguous()
         need = ctx.needs_input_grad
-        grad_x = ops.linear_fwd_dense(grad_y, w) if need[0] else None  # grad_y W^T of W [K, N]
+        # grad_y W^T of W [K, N]
+        grad_x = ops.linear_fwd_dense(grad_y, w, tiled=True) if need[0] else None
         grad_pal = grad_logits = grad_bias = None
         if need[1] or need[2]:
             grad_logits, grad_pal = ops.soft_ref_bwd(xc, grad_y, lg, pal, ctx.group_size,

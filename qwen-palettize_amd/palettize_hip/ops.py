@@ -151,18 +151,17 @@ def _lora_pair(a, b, first: str, second: str, rows_a: int, rows_b: int):
 
 
 def lut_linear_staged(M: int, N: int, K: int) -> bool:
-    """True when the library runs the hard forward / grad_x at this size by dequantising W into
-    the workspace and running the dense GEMM (its workspace query then asks for the bf16 W)."""
-    return (query("plz_lut_linear_fwd_workspace", M, N, K) >
-            query("plz_linear_fwd_dense_workspace", M, N, K))
+    """True when the hard forward at this size is fastest with W dequantised once and a dense GEMM
+    on it (grad_x: lut_linear_staged(M, K, N))."""
+    return query("plz_lut_linear_staged", M, N, K) != 0
 
 
 def lut_linear_fwd(x, packed, palette, bias=None, lora_t=None, lora_b=None, staged=True):
     """y = x W^T (+ bias) (+ lora_t lora_b^T).
 
-    staged: give the workspace the query asks for, so that from 4096 rows W is dequantised
-    into it and the dense GEMM runs on it; False keeps the one-pass LUT GEMM (workspace for
-    its tail partials only)."""
+    staged: dequantise W and run a dense GEMM on it where that is faster (lut_linear_staged; from
+    4096 rows inside the call, in the workspace that its query asks for); False keeps the
+    one-pass LUT GEMM (workspace for its tail partials only)."""
     N, K = _wshape(packed, palette)
     _need(x, "x", torch.bfloat16, 2)
     M = x.shape[0]
@@ -170,6 +169,8 @@ def lut_linear_fwd(x, packed, palette, bias=None, lora_t=None, lora_b=None, stag
         raise ValueError(f"x has {x.shape[1]} columns, W has K={K}")
     _bias(bias, N)
     rank = _lora_pair(lora_t, lora_b, "lora_t", "lora_b", M, N)
+    if staged and query("plz_lut_linear_staged", M, N, K) == 1:
+        return linear_fwd_dense(x, dequant(packed, palette), bias, lora_t, lora_b, tiled=True)
     y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     q = "plz_lut_linear_fwd_workspace" if staged else "plz_linear_fwd_dense_workspace"
     ws = _opt_workspace(query(q, M, N, K), x.device)
@@ -181,9 +182,9 @@ def lut_linear_fwd(x, packed, palette, bias=None, lora_t=None, lora_b=None, stag
 def lut_linear_bwd_x(grad_y, packed, palette, lora_gt=None, lora_a=None, staged=True):
     """grad_x = grad_y W (+ lora_gt lora_a).
 
-    staged: give the workspace the query asks for, so that from 4096 rows W is dequantised
-    into it and the dense GEMM runs on it; False keeps the one-pass LUT GEMM (workspace for
-    its tail partials only)."""
+    staged: dequantise W and run a dense GEMM on it where that is faster (lut_linear_staged; from
+    4096 rows inside the call, in the workspace that its query asks for); False keeps the
+    one-pass LUT GEMM (workspace for its tail partials only)."""
     N, K = _wshape(packed, palette)
     _need(grad_y, "grad_y", torch.bfloat16, 2)
     M = grad_y.shape[0]
@@ -198,6 +199,8 @@ def lut_linear_bwd_x(grad_y, packed, palette, lora_gt=None, lora_a=None, staged=
         rank = lora_gt.shape[1]
         if lora_gt.shape[0] != M or tuple(lora_a.shape) != (rank, K):
             raise ValueError("lora_gt / lora_a shape mismatch")
+    if staged and query("plz_lut_linear_staged", M, K, N) == 1:
+        return linear_bwd_x_dense(grad_y, dequant(packed, palette), lora_gt, lora_a, tiled=True)
     gx = torch.empty((M, K), dtype=torch.bfloat16, device=grad_y.device)
     q = "plz_lut_linear_bwd_x_workspace" if staged else "plz_linear_bwd_x_dense_workspace"
     ws = _opt_workspace(query(q, M, N, K), grad_y.device)
@@ -320,10 +323,11 @@ def linear_fwd_dense_swiglu_cat(x, w, lora_t=None, lora_b=None, keep_pre=True):
     return y, h
 
 
-def linear_fwd_dense(x, w, bias=None, lora_t=None, lora_b=None, residual=None):
+def linear_fwd_dense(x, w, bias=None, lora_t=None, lora_b=None, residual=None, tiled=False):
     """y = x w^T (+ bias) (+ lora_t lora_b^T); with residual (bf16 [M, N]) y = residual + that,
     added in the GEMM's epilogue with the rounding of a separate bf16 add
-    (plz_linear_fwd_dense_residual)."""
+    (plz_linear_fwd_dense_residual). tiled: on whichever GEMM core is the faster one for the shape
+    (plz_linear_fwd_tiled), whose sums over K may run in another order."""
     _need(x, "x", torch.bfloat16, 2)
     _need(w, "w", torch.bfloat16, 2)
     M, K = x.shape
@@ -333,11 +337,17 @@ def linear_fwd_dense(x, w, bias=None, lora_t=None, lora_b=None, residual=None):
     _bias(bias, N)
     rank = _lora_pair(lora_t, lora_b, "lora_t", "lora_b", M, N)
     y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    ws = _opt_workspace(query("plz_linear_fwd_dense_workspace", M, N, K), x.device)
     if residual is not None:
         _need(residual, "residual", torch.bfloat16, 2)
         if tuple(residual.shape) != (M, N):
             raise ValueError(f"residual must be [M, N] = [{M}, {N}]")
+    if tiled:
+        ws = _opt_workspace(query("plz_linear_tiled_workspace", M, N, K), x.device)
+        call("plz_linear_fwd_tiled", _ptr(x), _ptr(w), _ptr(bias), _ptr(lora_t), _ptr(lora_b),
+             rank, _ptr(residual), _ptr(y), _ptr(ws), _numel(ws), M, N, K, _stream(x))
+        return y
+    ws = _opt_workspace(query("plz_linear_fwd_dense_workspace", M, N, K), x.device)
+    if residual is not None:
         call("plz_linear_fwd_dense_residual", _ptr(x), _ptr(w), _ptr(bias), _ptr(lora_t),
              _ptr(lora_b), rank, _ptr(residual), _ptr(y), _ptr(ws), _numel(ws), M, N, K,
              _stream(x))
@@ -357,13 +367,14 @@ def linear_fwd_dense_kn(x, w, bias=None):
         raise ValueError("x / w shape mismatch")
     _bias(bias, N)
     y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    ws = _opt_workspace(query("plz_linear_bwd_x_dense_workspace", M, K, N), x.device)
+    ws = _opt_workspace(query("plz_linear_tiled_workspace", M, N, K), x.device)
     call("plz_linear_fwd_dense_kn", _ptr(x), _ptr(w), _ptr(bias), _ptr(y), _ptr(ws), _numel(ws), M,
          N, K, _stream(x))
     return y
 
 
-def linear_bwd_x_dense(grad_y, w, lora_gt=None, lora_a=None):
+def linear_bwd_x_dense(grad_y, w, lora_gt=None, lora_a=None, tiled=False):
+    """grad_x = grad_y w (+ lora_gt lora_a); tiled as in linear_fwd_dense."""
     _need(grad_y, "grad_y", torch.bfloat16, 2)
     _need(w, "w", torch.bfloat16, 2)
     M, N = grad_y.shape
@@ -380,6 +391,11 @@ def linear_bwd_x_dense(grad_y, w, lora_gt=None, lora_a=None):
         if lora_gt.shape[0] != M or tuple(lora_a.shape) != (rank, K):
             raise ValueError("lora_gt / lora_a shape mismatch")
     gx = torch.empty((M, K), dtype=torch.bfloat16, device=grad_y.device)
+    if tiled:
+        ws = _opt_workspace(query("plz_linear_tiled_workspace", M, K, N), grad_y.device)
+        call("plz_linear_bwd_x_tiled", _ptr(grad_y), _ptr(w), _ptr(lora_gt), _ptr(lora_a), rank,
+             _ptr(gx), _ptr(ws), _numel(ws), M, N, K, _stream(grad_y))
+        return gx
     ws = _opt_workspace(query("plz_linear_bwd_x_dense_workspace", M, N, K), grad_y.device)
     call("plz_linear_bwd_x_dense", _ptr(grad_y), _ptr(w), _ptr(lora_gt), _ptr(lora_a), rank,
          _ptr(gx), _ptr(ws), _numel(ws), M, N, K, _stream(grad_y))

@@ -172,7 +172,7 @@ class _LoRAFunction(torch.autograd.Function):
         a_rk = A.t().contiguous()          # [r, K]
         b_nr = B.contiguous()              # [N, r]
         t = ops.lora_project(x, a_rk, scale)   # s * x A   [M, r]
-        y = ops.linear_fwd_dense(t, b_nr, residual=residual)  # t B^T (+ residual)  [M, N]
+        y = ops.linear_fwd_dense(t, b_nr, residual=residual, tiled=True)  # t B^T (+ residual) [M, N]
         ctx.save_for_backward(x, a_rk, b_nr, t)
         ctx.scale = scale
         return y
@@ -183,6 +183,7 @@ class _LoRAFunction(torch.autograd.Function):
         x, a_rk, b_nr, t = ctx.saved_tensors
         gy = gy.contiguous()
         gt = ops.lora_grad_t(gy, b_nr, ctx.scale)            # s * gy B   [M, r]
-        gx = ops.linear_bwd_x_dense(gt, a_rk) if ctx.needs_input_grad[0] else None  # gt A^T
+        # gt A^T
+        gx = ops.linear_bwd_x_dense(gt, a_rk, tiled=True) if ctx.needs_input_grad[0] else None
         ga, gb = ops.lora_weight_grads(x, gy, t, gt, 1.0, out_dtype=torch.bfloat16)
         return gx, ga.t(), gb, None, gy if ctx.needs_input_grad[4] else None

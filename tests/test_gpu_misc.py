@@ -346,3 +346,36 @@ def test_dense_swiglu_epilogue(dev, M, N, K):
     assert ops.query("plz_linear_fwd_dense_workspace", M, N, K) == 0
     ref = ops.swiglu_fwd(ops.linear_fwd_dense(xd, wgd), ops.linear_fwd_dense(xd, wud))
     assert torch.equal(h, ref)
+
+
+@pytest.mark.parametrize("M,N,K,rank", [(65, 8, 64, 0), (100, 136, 520, 8), (129, 1032, 1000, 64),
+                                        (640, 1024, 2568, 16), (1000, 4096, 136, 32),
+                                        (70, 2560, 4096, 0), (1, 8, 8, 8)])
+def test_dense_gemms_of_few_tiles(dev, M, N, K, rank):
+    """The dense GEMMs at the sizes of the 128x128 core: ragged rows, columns and reductions (none,
+    one and several whole stages, a partial one), unsplit and split reductions, the rank segment,
+    bias and residual; without a workspace the unsplit launch."""
+    x, gy = randn_bf16(M, K, seed=1).to(dev), randn_bf16(M, N, seed=2).to(dev)
+    w = randn_bf16(N, K, seed=3, std=0.05).to(dev)
+    bias, res = randn_bf16(N, seed=4).to(dev), randn_bf16(M, N, seed=5).to(dev)
+    t = randn_bf16(M, rank, seed=6).to(dev) if rank else None
+    b = randn_bf16(N, rank, seed=7, std=0.1).to(dev) if rank else None
+    a = randn_bf16(rank, K, seed=8, std=0.1).to(dev) if rank else None
+    want = x.double() @ w.double().T + bias.double()
+    gwant = gy.double() @ w.double()
+    if rank:
+        want += t.double() @ b.double().T
+        gwant += t.double() @ a.double()
+    y = ops.linear_fwd_dense(x, w, bias, t, b, tiled=True)
+    assert_close(f32(y), want.cpu().numpy(), what="dense fwd")
+    yr = ops.linear_fwd_dense(x, w, bias, t, b, residual=res, tiled=True)
+    assert torch.equal(yr, y + res)
+    assert_close(f32(ops.linear_bwd_x_dense(gy, w, t, a, tiled=True)), gwant.cpu().numpy(), what="dense grad_x")
+    assert_close(f32(ops.linear_fwd_dense_kn(gy, w)), (gy.double() @ w.double()).cpu().numpy(),
+                 what="dense kn")
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    s = torch.cuda.current_stream().cuda_stream
+    ops.call("plz_linear_fwd_tiled", x.data_ptr(), w.data_ptr(), bias.data_ptr(),
+             t.data_ptr() if rank else None, b.data_ptr() if rank else None, rank, None,
+             out.data_ptr(), None, 0, M, N, K, s)
+    assert_close(f32(out), want.cpu().numpy(), what="dense fwd without a workspace")
