@@ -70,6 +70,24 @@ def test_attn_bwd_matches_fp32(dev, B, S, Hq, Hkv, std):
     assert all(torch.equal(a, b) for a, b in zip((gq, gk, gv), again)), "backward must be deterministic"
 
 
+@pytest.mark.parametrize("B,S,Hq,Hkv", [(4, 384, 6, 2), (8, 256, 1, 1), (2, 128, 32, 4),
+                                        (24, 128, 2, 1)])
+def test_attn_item_map_of_whole_xcds(dev, B, S, Hq, Hkv):
+    """(batch, kv head) pairs that divide by 8 are spread over the XCDs: bit for bit what each
+    sequence gives by itself (fewer pairs, plain order)."""
+    q, k, v = (t.to(dev) for t in _inputs(B, S, Hq, Hkv, seed=3 * S + Hq))
+    go = torch.randn(B, S, Hq, 128, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
+    go = go.to(dev)
+    o, lse = ops.attn_fwd(q, k, v)
+    grads = ops.attn_bwd(q, k, v, o, lse, go)
+    for b in range(B):
+        one = [t[b:b + 1].contiguous() for t in (q, k, v, go)]
+        ob, lb = ops.attn_fwd(*one[:3])
+        assert torch.equal(o[b:b + 1], ob) and torch.equal(lse[b:b + 1], lb)
+        for got, ref in zip(grads, ops.attn_bwd(*one[:3], ob, lb, one[3])):
+            assert torch.equal(got[b:b + 1], ref)
+
+
 def test_attn_bwd_layer_shape_sampled_heads(dev):
     """The layer's shape (seq 512, 32 query / 8 kv heads, batch 2): every gradient finite, and
     kv head 5 with its four query heads matches fp32 autograd."""
