@@ -337,9 +337,11 @@ def _soft_forward(ctx, x, palette, logits, bias, group_size, tau, noise, ste, se
     ctx.ref_seed = None
     hard = PLZ_W_HARD_PLAIN if semantics == "triton" else PLZ_W_HARD_NOISY
     if noise is None and _soft_in_reference_layout(x, palette, logits, N, K, group_size):
+        # dense, whatever the strides of the palette are (a plain clone keeps them)
+        pal = palette.detach().clone(memory_format=torch.contiguous_format)
+        xc, lg = x.contiguous(), logits.contiguous()
         # the reference's LCG draw, one seed per forward, in the kernels
         seed = _next_triton_step_seed() if semantics == "triton" else _next_soft_step_seed()
-        xc, lg, pal = x.contiguous(), logits.contiguous(), palette.detach().clone()
         w = ops.soft_ref_build_w(lg, pal, group_size, seed, float(tau),
                                  hard if ste else PLZ_W_SOFT, semantics)
         b = None if bias is None else bias.to(torch.bfloat16).contiguous()

@@ -271,3 +271,30 @@ def test_palette_expand_and_fold(dev, N, kg, GS, G, dt):
     eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dt]
     assert got.dtype == dt and bool(((got.double() - ref).abs() <=
                                      eps * ref.abs() + GS * kg * 2.0 ** -24 * mag + 1e-7).all())
+
+
+@pytest.mark.parametrize("semantics", ["cuda", "triton"])
+def test_soft_palette_of_other_strides(dev, semantics):
+    """A palette whose (G, 4) is the transpose of a dense (4, G), or every other row of one: the
+    same outputs, noise and gradients as the dense (G, 4)."""
+    M, K, N, GS = 33, 256, 1032, 256
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
+    logits = torch.randn(4, K, N, generator=g).to(torch.float16).to(dev)
+    dense = (torch.randn(-(-N // GS), 4, generator=g) * 0.02).to(torch.bfloat16).to(dev)
+    gy = torch.randn(M, N, generator=g).to(torch.bfloat16).to(dev)
+    spaced = torch.zeros(2 * dense.shape[0], 4, dtype=dense.dtype, device=dev)
+    spaced[::2] = dense
+    outs = []
+    for pal in (dense, dense.t().contiguous().t(), spaced[::2]):
+        FL._SOFT_STEP_SEED = FL._TRITON_STEP_SEED = 11
+        leaves = [x.clone().requires_grad_(True), pal.detach().requires_grad_(True),
+                  logits.clone().requires_grad_(True)]
+        y = FL.fused_lut_linear_soft(leaves[0], leaves[1], leaves[2], None, GS, 0.7,
+                                     semantics=semantics)
+        assert (FL._SOFT_STEP_SEED, FL._TRITON_STEP_SEED) == \
+            ((12, 11) if semantics == "cuda" else (11, 12))
+        outs.append([y, *torch.autograd.grad(y, leaves, gy)])
+    for other in outs[1:]:
+        for a, b, what in zip(outs[0], other, ("y", "grad_x", "grad_palette", "grad_logits")):
+            assert torch.equal(a, b), what
