@@ -275,6 +275,12 @@ int plz_soft_pw_ref_batched(const plz_pw_ref_desc* descs_device, int n, int64_t 
 int plz_soft_ref_build_w(const uint16_t* logits, int logits_dtype, const void* palette,
                          int palette_dtype, int64_t group_size, int triton_hash, uint32_t seed,
                          float tau, int mode, uint16_t* w, int64_t K, int64_t N, void* stream);
+/* The same, and the logits as the build read them into logits_copy (4, K, N), 8-byte aligned: for a
+ * backward that has to see the forward's values whatever is written to the logits in between. */
+int plz_soft_ref_build_w_copy(const uint16_t* logits, int logits_dtype, const void* palette,
+                              int palette_dtype, int64_t group_size, int triton_hash, uint32_t seed,
+                              float tau, int mode, uint16_t* w, uint16_t* logits_copy, int64_t K,
+                              int64_t N, void* stream);
 size_t plz_soft_ref_bwd_workspace(int64_t M, int64_t N, int64_t K);
 int plz_soft_ref_bwd(const uint16_t* x, const uint16_t* grad_y, const uint16_t* logits,
                      int logits_dtype, const void* palette, int palette_dtype, int64_t n_groups,

@@ -98,9 +98,11 @@ __device__ __forceinline__ void unpack_logits(const Weights& w, const uint2 (&v)
 // A workgroup covers 256 columns (4 per lane) and KR rows, its wave w rows w, w + 4, ...
 constexpr int KR = 32;
 
+// keep (optional): the logits as read
 template <bool ARITH>
 __global__ __launch_bounds__(256) void build_kernel(const Weights w, int mode,
-                                                    uint16_t* __restrict__ out) {
+                                                    uint16_t* __restrict__ out,
+                                                    uint16_t* __restrict__ keep) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t n = (int64_t)blockIdx.x * 256 + 4 * lane;
   if (n >= w.N) return;
@@ -114,6 +116,9 @@ __global__ __launch_bounds__(256) void build_kernel(const Weights w, int mode,
     const int64_t e = k * w.N + n;
     uint2 v[4];
     load_logits(w, e, v);
+    if (keep)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) *reinterpret_cast<uint2*>(keep + c * w.K * w.N + e) = v[c];
     float l[4][4];
     unpack_logits(w, v, l);
     uint32_t o[4];
@@ -329,23 +334,30 @@ int plz_palette_fold(const float* grad, void* out, int dtype, int64_t n_groups, 
   return check_launch("plz_palette_fold");
 }
 
-int plz_soft_ref_build_w(const uint16_t* logits, int logits_dtype, const void* palette,
-                         int palette_dtype, int64_t group_size, int triton_hash, uint32_t seed,
-                         float tau, int mode, uint16_t* w, int64_t K, int64_t N, void* stream) {
+int plz_soft_ref_build_w_copy(const uint16_t* logits, int logits_dtype, const void* palette,
+                              int palette_dtype, int64_t group_size, int triton_hash, uint32_t seed,
+                              float tau, int mode, uint16_t* w, uint16_t* logits_copy, int64_t K,
+                              int64_t N, void* stream) {
   const char* what = "plz_soft_ref_build_w";
   if (int rc = check(logits, logits_dtype, palette, palette_dtype, group_size, tau, K, N, what))
     return rc;
   PLZ_REQUIRE(mode == PLZ_W_SOFT || mode == PLZ_W_HARD_NOISY || mode == PLZ_W_HARD_PLAIN,
               "%s: unknown mode %d", what, mode);
-  PLZ_REQUIRE(w && ((uintptr_t)w & 7) == 0, "%s: w must be non-null, 8-byte aligned", what);
+  PLZ_REQUIRE(w && (((uintptr_t)w | (uintptr_t)logits_copy) & 7) == 0,
+              "%s: w must be non-null, w and logits_copy 8-byte aligned", what);
   const Weights g = {logits, palette, K, N, group_size, 1.f / tau, seed,
                      logits_dtype == PLZ_DT_FP16, palette_dtype};
   const dim3 grid((unsigned)((N + 255) / 256), (unsigned)row_blocks(K));
-  if (triton_hash)
-    hipLaunchKernelGGL(build_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, g, mode, w);
-  else
-    hipLaunchKernelGGL(build_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, g, mode, w);
+  auto kern = triton_hash ? build_kernel<true> : build_kernel<false>;
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, g, mode, w, logits_copy);
   return check_launch(what);
+}
+
+int plz_soft_ref_build_w(const uint16_t* logits, int logits_dtype, const void* palette,
+                         int palette_dtype, int64_t group_size, int triton_hash, uint32_t seed,
+                         float tau, int mode, uint16_t* w, int64_t K, int64_t N, void* stream) {
+  return plz_soft_ref_build_w_copy(logits, logits_dtype, palette, palette_dtype, group_size,
+                                   triton_hash, seed, tau, mode, w, nullptr, K, N, stream);
 }
 
 size_t plz_soft_ref_bwd_workspace(int64_t M, int64_t N, int64_t K) {

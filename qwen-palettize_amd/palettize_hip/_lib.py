@@ -94,6 +94,8 @@ SIGNATURES: dict[str, tuple] = {
     "plz_pw_ref_plan": (i64, [C.POINTER(PwRefDesc), i32, i64]),
     "plz_soft_pw_ref_batched": (i32, [p, i32, i64, i64, f32, u32, p]),
     "plz_soft_ref_build_w": (i32, [p, i32, p, i32, i64, i32, u32, f32, i32, p, i64, i64, p]),
+    "plz_soft_ref_build_w_copy": (i32, [p, i32, p, i32, i64, i32, u32, f32, i32, p, p, i64, i64,
+                                        p]),
     "plz_soft_ref_bwd_workspace": (sz, [i64, i64, i64]),
     "plz_soft_ref_bwd": (i32, [p, p, p, i32, p, i32, i64, i64, i32, u32, f32, i32, p, p, p, sz,
                                i64, i64, i64, p]),

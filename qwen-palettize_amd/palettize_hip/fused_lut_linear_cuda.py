@@ -339,14 +339,24 @@ def _soft_forward(ctx, x, palette, logits, bias, group_size, tau, noise, ste, se
     if noise is None and _soft_in_reference_layout(x, palette, logits, N, K, group_size):
         # dense, whatever the strides of the palette are (a plain clone keeps them)
         pal = palette.detach().clone(memory_format=torch.contiguous_format)
-        xc, lg = x.contiguous(), logits.contiguous()
+        xc, lg, copy, keep = x.contiguous(), logits.contiguous(), None, (None, None, None)
+        if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
+            # The backward draws P again, so it keeps what the forward read and not the caller's
+            # tensors, which an optimizer may write in between: the build writes the logits out
+            # (2560 x 4096: 53.3 -> 54.3 us, where a copy of its own takes 23.7). x, too, is a
+            # copy at the sizes where the native layout pads it.
+            if lg.data_ptr() == logits.data_ptr():
+                copy = torch.empty_like(lg)
+            if K % 256 and xc.data_ptr() == x.data_ptr():
+                xc = xc.clone()
+            keep = (xc, pal, lg if copy is None else copy)
         # the reference's LCG draw, one seed per forward, in the kernels
         seed = _next_triton_step_seed() if semantics == "triton" else _next_soft_step_seed()
         w = ops.soft_ref_build_w(lg, pal, group_size, seed, float(tau),
-                                 hard if ste else PLZ_W_SOFT, semantics)
+                                 hard if ste else PLZ_W_SOFT, semantics, copy)
         b = None if bias is None else bias.to(torch.bfloat16).contiguous()
         y = ops.linear_fwd_dense_kn(xc, w, b)
-        ctx.save_for_backward(xc, pal, lg, w)
+        ctx.save_for_backward(*keep, w)
         ctx.ref_seed, ctx.semantics = seed, semantics
         return y
     xp = _prep_x(x, K)

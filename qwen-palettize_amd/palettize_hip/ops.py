@@ -520,15 +520,19 @@ def _soft_ref_shapes(logits, palette, group_size):
 
 
 def soft_ref_build_w(logits, palette, group_size: int, seed: int, tau: float, mode: int,
-                     variant: str = "cuda"):
+                     variant: str = "cuda", copy=None):
     """W [K, N] bf16 of reference-layout logits (4, K, N) and palette (G, 4), the LCG noise of
     gumbel_lcg(variant=...) drawn in the kernel: the transpose of what soft_build_w makes of the
-    native-layout tensors. K and N multiples of 8."""
+    native-layout tensors. K and N multiples of 8. copy (like logits): the logits as read."""
     K, N = _soft_ref_shapes(logits, palette, group_size)
+    if copy is not None:
+        _need(copy, "copy", logits.dtype, 3)
+        if copy.shape != logits.shape:
+            raise ValueError("copy must have the logits' shape")
     w = torch.empty((K, N), dtype=torch.bfloat16, device=logits.device)
-    call("plz_soft_ref_build_w", _ptr(logits), _DT[logits.dtype], _ptr(palette),
+    call("plz_soft_ref_build_w_copy", _ptr(logits), _DT[logits.dtype], _ptr(palette),
          _DT[palette.dtype], int(group_size), int(variant == "triton"), int(seed) & 0xFFFFFFFF,
-         float(tau), int(mode), _ptr(w), K, N, _stream(logits))
+         float(tau), int(mode), _ptr(w), _ptr(copy), K, N, _stream(logits))
     return w
 
 

@@ -298,3 +298,33 @@ def test_soft_palette_of_other_strides(dev, semantics):
     for other in outs[1:]:
         for a, b, what in zip(outs[0], other, ("y", "grad_x", "grad_palette", "grad_logits")):
             assert torch.equal(a, b), what
+
+
+@pytest.mark.parametrize("K", [512, 264])
+@pytest.mark.parametrize("write", ["in place", "data"])
+@pytest.mark.parametrize("train", [(0, 1, 2), (1,), (0,)], ids=["all", "palette", "x"])
+def test_inputs_written_between_the_soft_forward_and_its_backward(dev, K, write, train):
+    """The backward belongs to the forward's values: logits, palette and (at a K that is not a
+    multiple of 256) x written after the forward, with or without torch's version counter seeing
+    it, change none of its gradients."""
+    M, N, GS = 40, 520, 256
+    g = torch.Generator().manual_seed(K)
+    vals = [torch.randn(M, K, generator=g).to(torch.bfloat16),
+            (torch.randn(-(-N // GS), 4, generator=g) * 0.02).to(torch.bfloat16),
+            torch.randn(4, K, N, generator=g).to(torch.float16)]
+    gy = torch.randn(M, N, generator=g).to(torch.bfloat16).to(dev)
+    grads = []
+    for touch in (False, True):
+        FL._SOFT_STEP_SEED = 30
+        leaves = [v.to(dev).requires_grad_(i in train) for i, v in enumerate(vals)]
+        y = FL.fused_lut_linear_soft(leaves[0], leaves[1], leaves[2], None, GS, 0.7)
+        if touch:
+            for t in leaves if K % 256 else leaves[1:]:
+                if write == "data":
+                    t.data.mul_(-3.0)
+                else:
+                    with torch.no_grad():
+                        t.mul_(-3.0)
+        grads.append(torch.autograd.grad(y, [leaves[i] for i in train], gy))
+    for a, b, i in zip(*grads, train):
+        assert torch.equal(a, b), ("grad_x", "grad_palette", "grad_logits")[i]
