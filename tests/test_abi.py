@@ -145,6 +145,43 @@ def test_dropin_layout_maps_match_oracle():
     assert torch.count_nonzero(nk4[:, K:, :]) == 0
 
 
+def test_palette_helpers_keep_type_and_gradient():
+    """palette_from_reference is differentiable; palette_grad_to_reference takes any float type and
+    strides and answers in the gradient's type."""
+    from palettize_hip import fused_lut_linear_cuda as FL
+    _palette_helpers(FL, torch.device("cpu"))
+
+
+def _palette_helpers(FL, device):
+    g = torch.Generator().manual_seed(1)
+    N, K, GS, G = 520, 512, 256, 4
+    up = torch.randn(N, 2, 4, generator=g).to(device)
+    for dt in (torch.float32, torch.bfloat16, torch.float64):
+        pal = torch.randn(G, 4, generator=g).to(dt).to(device).requires_grad_(True)
+        nat = FL.palette_from_reference(pal, N, K, GS)
+        assert nat.dtype == torch.float32 and nat.requires_grad
+        got, = torch.autograd.grad(nat, pal, up)
+        want = torch.zeros(G, 4, dtype=torch.float64)
+        want.index_add_(0, torch.arange(N) // GS, up.cpu().double().sum(1))
+        # fp32 sums of 512 terms, rounded to the palette's type
+        eps = max(torch.finfo(dt).eps, 2.0 ** -14)
+        assert got.dtype == dt
+        assert torch.allclose(got.cpu().double(), want, rtol=eps, atol=1e-3)
+    grad = torch.randn(N, 2, 4, generator=g, dtype=torch.float64).to(device)
+    want = torch.zeros(G, 4, dtype=torch.float64)
+    want.index_add_(0, torch.arange(N) // GS, grad.cpu().sum(1))
+    out = FL.palette_grad_to_reference(grad, GS, G)
+    assert out.dtype == torch.float64 and torch.allclose(out.cpu(), want)
+    f = grad.float().requires_grad_(True)
+    for strided in (f.transpose(0, 1).contiguous().transpose(0, 1), f[::2], f.half()):
+        out = FL.palette_grad_to_reference(strided, GS)
+        ref = torch.zeros(out.shape, dtype=torch.float64)
+        ref.index_add_(0, torch.arange(strided.shape[0]) // GS,
+                       strided.detach().cpu().double().sum(1))
+        assert out.dtype == strided.dtype and out.requires_grad
+        assert torch.allclose(out.detach().cpu().double(), ref, rtol=2e-2, atol=5e-2)
+
+
 def test_attention_argument_errors(lib):
     """Shape, support and workspace checks of the attention entry points fail before any GPU
     work (pointer 16 stands for an aligned device pointer and is never dereferenced)."""

@@ -262,15 +262,17 @@ def test_palette_expand_and_fold(dev, N, kg, GS, G, dt):
     pal = torch.randn(G, 4, generator=g).to(dt).to(dev)
     want = pal.float().repeat_interleave(GS, 0)[:N][:, None].expand(N, kg, 4)
     assert torch.equal(FL.palette_from_reference(pal, N, 256 * kg, GS), want)
+    assert torch.equal(FL._expand_palette(pal, N, 256 * kg, GS), want)
     grad = torch.randn(N, kg, 4, generator=g).to(dev)
-    got = FL.palette_grad_to_reference(grad, GS, G, dt)
     ref, mag = (torch.zeros(G, 4, dtype=torch.float64, device=dev) for _ in range(2))
     rows = torch.arange(N, device=dev) // GS
     ref.index_add_(0, rows, grad.double().sum(1))
     mag.index_add_(0, rows, grad.double().abs().sum(1))
     eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dt]
-    assert got.dtype == dt and bool(((got.double() - ref).abs() <=
-                                     eps * ref.abs() + GS * kg * 2.0 ** -24 * mag + 1e-7).all())
+    for fold in (FL._fold_palette_grad, FL.palette_grad_to_reference):
+        got = fold(grad, GS, G, dt)
+        assert got.dtype == dt and bool(((got.double() - ref).abs() <=
+                                         eps * ref.abs() + GS * kg * 2.0 ** -24 * mag + 1e-7).all())
 
 
 @pytest.mark.parametrize("semantics", ["cuda", "triton"])
@@ -328,3 +330,9 @@ def test_inputs_written_between_the_soft_forward_and_its_backward(dev, K, write,
         grads.append(torch.autograd.grad(y, [leaves[i] for i in train], gy))
     for a, b, i in zip(*grads, train):
         assert torch.equal(a, b), ("grad_x", "grad_palette", "grad_logits")[i]
+
+
+def test_palette_helpers_keep_type_and_gradient_on_the_gpu(dev):
+    """The same calls as on the CPU (test_abi.py), with the same types and gradients."""
+    from test_abi import _palette_helpers
+    _palette_helpers(FL, dev)
