@@ -151,15 +151,21 @@ class QwenLoRA(nn.Module):
         y_base = self.base(x)
         lead = x.shape[:-1]
         x_flat = x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
-        if (y_base.is_cuda and y_base.dtype == torch.bfloat16 and y_base.is_contiguous()
-                and tuple(y_base.shape) == (*lead, self.lora_B.shape[0])
-                and y_base.numel() > 0 and y_base.data_ptr() % 16 == 0):
+        if _adds_in_epilogue(y_base, x_flat, (*lead, self.lora_B.shape[0])):
             # the add rides in the epilogue of the t B^T GEMM, rounded as a separate add would be
             y = _LoRAFunction.apply(x_flat, self.lora_A, self.lora_B, self.scaling,
                                     y_base.reshape(-1, y_base.shape[-1]))
             return y.reshape(y_base.shape)
         lora = _LoRAFunction.apply(x_flat, self.lora_A, self.lora_B, self.scaling, None)
         return y_base + lora.reshape(*lead, -1).to(y_base.dtype)
+
+
+def _adds_in_epilogue(y_base, x, shape):
+    """True where the GEMM kernel may read the base output itself: on x's device (a tensor of
+    another one is left to torch's add, which refuses it), dense, aligned bf16 of the very shape."""
+    return (y_base.is_cuda and y_base.device == x.device and y_base.dtype == torch.bfloat16
+            and y_base.is_contiguous() and tuple(y_base.shape) == shape
+            and y_base.numel() > 0 and y_base.data_ptr() % 16 == 0)
 
 
 class _LoRAFunction(torch.autograd.Function):

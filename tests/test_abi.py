@@ -182,6 +182,25 @@ def _palette_helpers(FL, device):
         assert torch.allclose(out.detach().cpu().double(), ref, rtol=2e-2, atol=5e-2)
 
 
+def test_lora_epilogue_reads_only_base_outputs_of_its_own_device():
+    """The residual that QwenLoRA hands to the GEMM kernel as a pointer (stand-ins for GPU tensors:
+    the rule looks at these properties only)."""
+    from types import SimpleNamespace
+    from palettize_hip.qwen_model import _adds_in_epilogue
+
+    def tensor(device="cuda:0", shape=(2, 8), dtype=torch.bfloat16, dense=True, at=256):
+        return SimpleNamespace(is_cuda=device != "cpu", device=torch.device(device), dtype=dtype,
+                               shape=shape, is_contiguous=lambda: dense,
+                               numel=lambda: int(np.prod(shape)), data_ptr=lambda: at)
+
+    x = tensor(shape=(2, 16))
+    assert _adds_in_epilogue(tensor(), x, (2, 8))
+    for other in (tensor("cuda:1"), tensor("cpu"), tensor(shape=(2, 9)), tensor(at=8),
+                  tensor(dtype=torch.float32), tensor(dense=False)):
+        assert not _adds_in_epilogue(other, x, (2, 8))
+    assert not _adds_in_epilogue(tensor(shape=(0, 8)), x, (0, 8))
+
+
 def test_attention_argument_errors(lib):
     """Shape, support and workspace checks of the attention entry points fail before any GPU
     work (pointer 16 stands for an aligned device pointer and is never dereferenced)."""
