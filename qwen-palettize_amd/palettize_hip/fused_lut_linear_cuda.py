@@ -146,11 +146,27 @@ def _expand_palette(palette: Tensor, N: int, K: int, group_size: int) -> Tensor:
     return palette_from_reference(palette, N, K, group_size)
 
 
+# A group is folded by one workgroup, which is slow for many entries: with its host side 6.4 us at 10
+# thousand, 9.8 / 12.9 / 18.8 / 22.1 / 64.9 at 68 / 97 / 156 / 185 / 370 thousand (one palette for a
+# whole weight). Two folds, the first of parts of about 2^13 entries, take 13.4-14.9 (torch's two
+# sums 16.1-18.5): the line is at 2^17.
+_FOLD_ENTRIES = 1 << 17
+_FOLD_PART = 1 << 13
+
+
 def _fold_palette_grad(grad: Tensor, group_size: int, n_groups: int, dtype: torch.dtype) -> Tensor:
     """palette_grad_to_reference of the kernels' dense fp32 gradient, likewise (11.6 us, 16.8)."""
-    if dtype in ops._DT and grad.numel() > 0:
-        return ops.palette_fold(grad, n_groups, group_size, dtype)
-    return palette_grad_to_reference(grad, group_size, n_groups, dtype)
+    if dtype not in ops._DT or grad.numel() == 0:
+        return palette_grad_to_reference(grad, group_size, n_groups, dtype)
+    N, kg = grad.shape[0], grad.shape[1]
+    if min(group_size, N) * kg > _FOLD_ENTRIES:
+        # rows of a part: parts end where groups end, unless there is only one group
+        part = max(1, _FOLD_PART // kg)
+        if group_size < N:
+            part = next(r for r in range(part, 0, -1) if group_size % r == 0)
+        grad = ops.palette_fold(grad, -(-N // part), part).unsqueeze(1)
+        group_size = grad.shape[0] if group_size >= N else group_size // part
+    return ops.palette_fold(grad, n_groups, group_size, dtype)
 
 
 def _prep_x(x: Tensor, K: int) -> Tensor:

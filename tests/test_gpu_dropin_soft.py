@@ -336,3 +336,25 @@ def test_palette_helpers_keep_type_and_gradient_on_the_gpu(dev):
     """The same calls as on the CPU (test_abi.py), with the same types and gradients."""
     from test_abi import _palette_helpers
     _palette_helpers(FL, dev)
+
+
+@pytest.mark.parametrize("N,kg,GS,folds", [(9728, 38, 9728, 2), (9728, 13, 9728, 1),
+                                           (9728, 14, 9728, 2), (1024, 38, 1 << 20, 1),
+                                           (4096, 38, 1 << 20, 2), (9728, 38, 4864, 2),
+                                           (9000, 38, 4001, 2), (9728, 38, 2432, 1)])
+def test_large_palette_groups_are_folded_in_two_steps(dev, N, kg, GS, folds, monkeypatch):
+    """A group of more than 2^17 entries is folded in parts first (a lone group of any size, groups
+    with a last partial one, a prime number of rows): the fp64 sum up to n terms' rounding."""
+    calls = []
+    fold = ops.palette_fold
+    monkeypatch.setattr(ops, "palette_fold", lambda *a: calls.append(1) or fold(*a))
+    grad = torch.randn(N, kg, 4, generator=torch.Generator().manual_seed(kg)).to(dev)
+    G = -(-N // GS) + 1
+    got = FL._fold_palette_grad(grad, GS, G, torch.float32)
+    assert len(calls) == folds and got.shape == (G, 4)
+    ref, mag = (torch.zeros(G, 4, dtype=torch.float64, device=dev) for _ in range(2))
+    rows = torch.arange(N, device=dev) // GS
+    ref.index_add_(0, rows, grad.double().sum(1))
+    mag.index_add_(0, rows, grad.double().abs().sum(1))
+    n = min(GS, N) * kg
+    assert bool(((got.double() - ref).abs() <= n * 2.0 ** -24 * mag).all())
