@@ -26,6 +26,7 @@
 //   lookup words (8 B per row and stage). Words and lookup words go straight into registers,
 //   RD stages ahead; only the x slice goes through LDS.
 #include "plz_common.h"
+#include "plz_gemv_split.h"
 #include "palettize_hip.h"
 
 namespace plz {
@@ -627,12 +628,7 @@ __host__ __device__ inline uint32_t plane_word(uint32_t src_a, uint32_t src_b, i
   return o;
 }
 
-// x prep, one chunk per (linear d, stage s) of the workspace at (d * max_stages + s) * chunk:
-// A rows m = 2 t + piece, 256 B each (the fragments of both MFMA halves: 16-byte piece
-// c = 8 h + 2 j + half, holding stage k = 128 h + 64 half + 16 j + (0..15), stored at
-// c ^ (m & 15)); then the tokens' E8M0 scale bytes (16 B), their stage sums X as fp32 (64 B)
-// and 48 B of padding.
-__host__ __device__ constexpr int pl_chunk(int M) { return 512 * M + 128; }
+// x prep: chunk (d * max_stages + s) of the workspace holds linear d's stage s (pl_chunk)
 __host__ __device__ constexpr int pl_nx(int M) {
   return (pl_chunk(M) + WAVES * 1024 - 1) / (WAVES * 1024);
 }
@@ -1045,7 +1041,6 @@ __global__ void pack_planes_kernel(const uint32_t* __restrict__ packed, uint4* _
 // 13.5 / 18.6 / 19.3 -> 10.4 / 14.2 / 18.2, down 26.1 / 31.6 / 33.9 -> 10.9 / 12.8 / 17.1. (The
 // decode layout chains its MFMAs through one accumulator over all of K: splitting that needs
 // per-chunk sums in the streaming kernel too, which cost it 1.3% at M = 16.)
-constexpr int SP_WAVES = 16;  // most waves per workgroup
 // This workgroup's linear and its first row. Descriptors of up to 64 linears are searched with
 // one load per lane and a ballot (a binary search would chain its loads).
 template <bool GROUPED>
@@ -1078,19 +1073,11 @@ __device__ __forceinline__ plz_gemv_desc split_desc(const Table<GROUPED>& tb, in
 // token's piece (2 at M = 1). Every lane stores its elements, also those that hold no token: a
 // lane condition around the stores would let the compiler sink the MFMAs into it, where the
 // masked-off lanes' operands are missing.
-template <int NI>
-__host__ __device__ constexpr int sp_sum_bytes(int rbw) {  // plane sums and lookup words, a wave
-  return rbw * (3 * NI * 64 * 4 + 16 * 8);
-}
-template <int NI>
-__host__ __device__ constexpr int sp_wave_bytes(int rbw, int M) {
-  return sp_sum_bytes<NI>(rbw) + 2 * pl_chunk(M);
-}
 template <int NI, int RBW, bool GROUPED>
 __global__ __launch_bounds__(64 * SP_WAVES) void gemv_pl_split_kernel(
     const plz_gemv_desc* __restrict__ descs, int n_desc, plz_gemv_desc single, int M) {
   extern __shared__ uint4 smem[];
-  constexpr int NP = NI / 2, SB = sp_sum_bytes<NI>(RBW), LUT_OFF = RBW * 3 * NI * 64 * 4;
+  constexpr int NP = NI / 2, SB = sp_sum_bytes(NI, RBW), LUT_OFF = RBW * 3 * NI * 64 * 4;
   const Table<GROUPED> tb{descs, n_desc, single};
   int64_t row0;
   const plz_gemv_desc d = split_desc<GROUPED>(tb, 16 * RBW, row0);
@@ -1217,46 +1204,21 @@ __global__ __launch_bounds__(64 * SP_WAVES) void gemv_pl_split_kernel(
   if (folds && n < d.N) d.y[(int64_t)tok * d.N + n] = (uint16_t)f2bf(y0 + y1);
 }
 
-// Shape of a split launch: rbw row blocks (16 rows) per workgroup, 0 to stream, and its waves.
-struct SplitPlan {
-  int rbw, waves;
-};
-// most: the items (128 rows) up to which a split launch is the faster one; max_rbw: the kernel's
-// most row blocks; stages: of the longest linear, a wave takes one per pass.
-// Workgroups of 16 waves fill a CU at these register counts, so rbw is the least that leaves
-// one round of them, and a launch of more workgroups than CUs gets at most 8 waves each. Measured
-// on 2560 -> 9728 (76 items) at M = 1 / 4: 7.3 / 11.4 us in one round of 152 / 304 workgroups
-// of 10 waves, 8.1 / 9.2 us with 304 of 5.
-static SplitPlan split_plan(int64_t items, int64_t most, int max_rbw, int64_t stages) {
-  SplitPlan p{0, 0};
-  const int64_t cus = cu_count();
-  if (items > most) return p;
-  p.rbw = items * 8 <= cus ? 1 : items * 4 <= cus ? 2 : 4;
-  p.rbw = p.rbw < max_rbw ? p.rbw : max_rbw;
-  const int64_t cap = items * (8 / p.rbw) <= cus ? SP_WAVES : SP_WAVES / 2;
-  const int64_t passes = (stages + cap - 1) / cap;
-  p.waves = (int)((stages + passes - 1) / passes);
-  return p;
-}
 template <int NI, int RBW, bool GROUPED>
 static int launch_pl_split_r(int waves, int64_t items, hipStream_t st, const plz_gemv_desc* descs,
                              int n, plz_gemv_desc single, int M, const char* what) {
   auto kern = gemv_pl_split_kernel<NI, RBW, GROUPED>;
-  constexpr int kMost = 160 * 1024;
-  const int fit = kMost / sp_wave_bytes<NI>(RBW, M);
-  waves = waves < fit ? waves : fit;
-  waves = waves < RBW * NI / 2 ? RBW * NI / 2 : waves;  // the folds take RBW * NI / 2 waves
-  static_assert(RBW * NI / 2 * sp_wave_bytes<NI>(RBW, NI == 2 ? 1 : 8) <= kMost, "LDS");
+  static_assert(RBW * NI / 2 * sp_wave_bytes(NI, RBW, NI == 2 ? 1 : 8) <= SP_LDS, "LDS");
   static uint64_t lds_done = 0;
-  if (int rc = reserve_lds((const void*)kern, kMost, lds_done, what)) return rc;
+  if (int rc = reserve_lds((const void*)kern, SP_LDS, lds_done, what)) return rc;
   hipLaunchKernelGGL(kern, dim3((unsigned)(items * (8 / RBW))), dim3(64 * waves),
-                     (size_t)waves * sp_wave_bytes<NI>(RBW, M), st, descs, n, single, M);
+                     (size_t)waves * sp_wave_bytes(NI, RBW, M), st, descs, n, single, M);
   return check_launch(what);
 }
 template <int NI, bool GROUPED>
 static int launch_pl_split(SplitPlan p, int64_t items, hipStream_t st, const plz_gemv_desc* descs,
                            int n, plz_gemv_desc single, int M, const char* what) {
-  if constexpr (NI == 2)  // at M > 1 the plane sums of four row blocks leave LDS for too few waves
+  if constexpr (NI == 2)
     if (p.rbw == 4)
       return launch_pl_split_r<NI, 4, GROUPED>(p.waves, items, st, descs, n, single, M, what);
   if (p.rbw == 2)
@@ -1296,14 +1258,10 @@ template <bool GROUPED>
 static int launch_pl(int64_t items, hipStream_t st, const plz_gemv_desc* descs, int n,
                      plz_gemv_desc single, int M, int max_stages, uint8_t* ws, size_t ws_bytes,
                      const char* what) {
-  // up to one item per CU at M = 1 (240 items: 22.6 us against 27.9 streaming; 304 tie), where the
-  // x pieces are a sixteenth of the work; they are made once per workgroup, so from M = 2 up to
-  // 5/8 (152 items at M = 4 / 8: 14.0 / 18.0 us against 18.6 / 19.3; 240: 34 / 42 against 33 / 35)
-  const SplitPlan p =
-      split_plan(items, M == 1 ? cu_count() : cu_count() * 5 / 8, M == 1 ? 4 : 2, max_stages);
-  if (M <= 8 && p.rbw)
-    return M == 1 ? launch_pl_split<2, GROUPED>(p, items, st, descs, n, single, M, what)
-                  : launch_pl_split<4, GROUPED>(p, items, st, descs, n, single, M, what);
+  const SplitPlan p = split_plan_on(items, max_stages, M, cu_count());
+  if (p.rbw)
+    return M == 1 ? launch_pl_split<sp_ni(1), GROUPED>(p, items, st, descs, n, single, M, what)
+                  : launch_pl_split<sp_ni(8), GROUPED>(p, items, st, descs, n, single, M, what);
   if (M == 1)
     return launch_pl_nx<pl_nx(1), 1, 2, GROUPED>(items, st, descs, n, single, M, max_stages, ws,
                                                  ws_bytes, what);
