@@ -184,6 +184,8 @@ int plz_linear_fwd_dense_swiglu_cat(const uint16_t* x, const uint16_t* w, const 
  * 0 in one pass (plz_lut_linear_fwd / _bwd_x); 1 plz_dequant and a tiled GEMM below on the bf16 W;
  * 2 so too, which those entries do themselves in the workspace that their queries ask for. */
 int plz_lut_linear_staged(int64_t rows, int64_t outputs, int64_t reduction);
+/* The same for a forward whose bf16 W the grad_x of the same pass uses again. */
+int plz_lut_linear_staged_pair(int64_t M, int64_t N, int64_t K);
 /* plz_linear_fwd_dense (with an optional residual) and plz_linear_bwd_x_dense on the GEMM core,
  * 128x128 or 256x256 tiles, that is the faster one for the shape. Where that is the smaller one,
  * the fp32 sums over K (N) are split differently from the dense entries'. The workspace (optional:

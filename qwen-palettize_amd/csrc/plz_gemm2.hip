@@ -1711,6 +1711,19 @@ static bool staged_rows(int64_t I, int64_t J, int64_t R) {
   return I > sk::kMaxRows && dense_splits(I, J, R, &us) > 0 &&
          us + 2.9 + 0.385e-6 * (double)J * (double)R < 0.97 * core256_us(I, J, R, 1.55);
 }
+// ... for one GEMM by itself. Where W is wide (J > 3 R) the LUT core's few row tiles spread over many
+// columns, while the dense core reads a freshly written W from beyond the L2s, which costs more
+// than the models say once a CU holds two workgroups of it (short prefetch) or W is large: LUT
+// and dequantise + dense in us, 256 -> 9728 at M = 512 / 640 13.2 / 13.4 and 14.2 / 16.0; 1024 ->
+// 9728 at M = 128 / 256 / 640 28.7 / 28.6 / 28.5 and 28.4 / 24.9 / 34.6; 2560 -> 9728 at M = 128 /
+// 200 / 512 42.3 / 42.3 / 49.1 and 35.5 / 45.2 / 51.7. From 769 rows (2048 of 1024 -> 9728: 64.5 and
+// 56.2) and for 1280 -> 4864 (M = 640: 25.0 and 18.8) the models hold.
+static bool staged_alone(int64_t I, int64_t J, int64_t R) {
+  if (!staged_rows(I, J, R)) return false;
+  if (J <= 3 * R || I <= 128 || I > 768) return true;
+  const int64_t tiles = ((I + 127) / 128) * ((J + 127) / 128);  // of the 128x128 core
+  return tiles <= cu_count() && (I > 256 || J * R < ((int64_t)1 << 24));
+}
 // Tile-rows walked together by the dense GEMMs (consecutive workgroups share an x / grad_y
 // panel within groups of this many tile-rows). Measured on the hard step at M = 16384: 4 (and
 // 2, 6) 1085-1092 TFLOP/s against 1081 for 8, 1067-1069 for 16, 1053 for a column walk.
@@ -1975,7 +1988,14 @@ size_t plz_linear_fwd_dense_workspace(int64_t M, int64_t N, int64_t K) {
 
 int plz_lut_linear_staged(int64_t I, int64_t J, int64_t R) {
   if (I <= 0 || J <= 0 || R <= 0) return 0;
-  return I >= kStagedRows ? 2 : staged_rows(I, J, R) ? 1 : 0;
+  return I >= kStagedRows ? 2 : staged_alone(I, J, R) ? 1 : 0;
+}
+
+int plz_lut_linear_staged_pair(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  // grad_x would dequantise W anyway (2560 -> 9728 at M = 512, forward + grad_x: 91 us kept, 120 as
+  // two LUT GEMMs)
+  return M >= kStagedRows ? 2 : staged_rows(M, N, K) ? 1 : 0;
 }
 
 size_t plz_linear_tiled_workspace(int64_t M, int64_t N, int64_t K) {

@@ -37,7 +37,8 @@ class LUTLinearFunction(torch.autograd.Function):
         lora_a, lora_b = _c(lora_a), _c(lora_b)
         t = ops.lora_project(x, lora_a, lora_scale) if lora_a is not None else None
         w = None
-        if ops.lut_linear_staged(x.shape[0], packed.shape[0], x.shape[1]):
+        if ops.lut_linear_staged(x.shape[0], packed.shape[0], x.shape[1],
+                                 grad_x=ctx.needs_input_grad[0]):
             w = ops.dequant(packed, palette)
             y = ops.linear_fwd_dense(x, w, bias, t, lora_b, tiled=True)
             if not ctx.needs_input_grad[0]:

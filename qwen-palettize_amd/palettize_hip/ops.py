@@ -150,10 +150,11 @@ def _lora_pair(a, b, first: str, second: str, rows_a: int, rows_b: int):
     return r
 
 
-def lut_linear_staged(M: int, N: int, K: int) -> bool:
+def lut_linear_staged(M: int, N: int, K: int, grad_x: bool = False) -> bool:
     """True when the hard forward at this size is fastest with W dequantised once and a dense GEMM
-    on it (grad_x: lut_linear_staged(M, K, N))."""
-    return query("plz_lut_linear_staged", M, N, K) != 0
+    on it (grad_x by itself: lut_linear_staged(M, K, N)); grad_x: that W serves the pass's grad_x
+    too."""
+    return query("plz_lut_linear_staged_pair" if grad_x else "plz_lut_linear_staged", M, N, K) != 0
 
 
 def lut_linear_fwd(x, packed, palette, bias=None, lora_t=None, lora_b=None, staged=True):

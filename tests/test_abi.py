@@ -201,6 +201,25 @@ def test_lora_epilogue_reads_only_base_outputs_of_its_own_device():
     assert not _adds_in_epilogue(tensor(shape=(0, 8)), x, (0, 8))
 
 
+@pytest.mark.parametrize("M,J,R,staged", [
+    # one LUT GEMM of M x J outputs over R at both sides of the rule (256 CUs)
+    (48, 4096, 2560, 0), (128, 4096, 2560, 1), (1000, 4096, 2560, 1), (777, 9728, 2560, 0),
+    (4096, 9728, 2560, 2), (128, 9728, 2560, 1), (200, 9728, 2560, 0), (257, 9728, 2560, 1),
+    (385, 9728, 2560, 0), (512, 9728, 2560, 0), (640, 9728, 2560, 0), (512, 9728, 1024, 0),
+    (256, 9728, 1024, 1), (2048, 9728, 1024, 1), (640, 9728, 256, 0), (128, 9728, 256, 1),
+    (640, 4864, 1280, 1), (640, 3072, 1024, 1), (640, 2560, 9728, 1)])
+def test_lut_gemms_of_wide_outputs_stay_where_they_are_faster(lib, M, J, R, staged):
+    if torch.cuda.is_available() and \
+            torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes for 256 CUs")
+    assert lib.plz_lut_linear_staged(M, J, R) == staged
+    # with grad_x on the same W a wide forward is staged as any other
+    if 128 <= M <= 640:
+        assert lib.plz_lut_linear_staged_pair(M, J, R) == 1
+    else:
+        assert lib.plz_lut_linear_staged_pair(M, J, R) == staged
+
+
 def test_attention_argument_errors(lib):
     """Shape, support and workspace checks of the attention entry points fail before any GPU
     work (pointer 16 stands for an aligned device pointer and is never dereferenced)."""
