@@ -1323,23 +1323,26 @@ __global__ __launch_bounds__(TAIL_THREADS) void tail_reduce_kernel(const Args g)
     for (int tj = 0; tj < WT_J; ++tj)
 #pragma unroll
       for (int e = 0; e < 16; ++e) a[tl][tj][e] = 0.f;
-  for (int p = 0; p < g.tail_split; ++p) {
+  // a number of blocks that the compiler knows: with a test inside the loop the loads of a part wait
+  // for each other (whole tiles, 2560 -> 9728 at M = 512: 46.4 -> 48.5 us)
+  auto sum = [&](auto blocks) {
+    for (int p = 0; p < g.tail_split; ++p)
 #pragma unroll
-    for (int tl = 0; tl < 2; ++tl) {
-      if (tl >= live) break;
+      for (int tl = 0; tl < decltype(blocks)::value; ++tl)
 #pragma unroll
-      for (int tj = 0; tj < WT_J; ++tj)
+        for (int tj = 0; tj < WT_J; ++tj)
 #pragma unroll
-        for (int e4 = 0; e4 < 4; ++e4) {
-          const float4 v = src[(int64_t)p * (TILE * TILE / 4) +
-                               (((ti0 + tl) * WT_J + tj) * 4 + e4) * NTHR + gt];
-          a[tl][tj][4 * e4] += v.x;
-          a[tl][tj][4 * e4 + 1] += v.y;
-          a[tl][tj][4 * e4 + 2] += v.z;
-          a[tl][tj][4 * e4 + 3] += v.w;
-        }
-    }
-  }
+          for (int e4 = 0; e4 < 4; ++e4) {
+            const float4 v = src[(int64_t)p * (TILE * TILE / 4) +
+                                 (((ti0 + tl) * WT_J + tj) * 4 + e4) * NTHR + gt];
+            a[tl][tj][4 * e4] += v.x;
+            a[tl][tj][4 * e4 + 1] += v.y;
+            a[tl][tj][4 * e4 + 2] += v.z;
+            a[tl][tj][4 * e4 + 3] += v.w;
+          }
+  };
+  if (live == 2) sum(std::integral_constant<int, 2>{});
+  else if (live == 1) sum(std::integral_constant<int, 1>{});
   // bf16 (alpha * acc + bias) of the slab's 64 rows in LDS, as stage_tile_bf16 computes it
 #pragma unroll
   for (int tj = 0; tj < WT_J; ++tj) {

@@ -411,16 +411,26 @@ def test_lut_linear_fwd_few_rows(dev, M, N, K, rank, bias):
     assert_close(f32(y), want, what=f"few-row fwd M={M} N={N} K={K} rank={rank}")
 
 
-@pytest.mark.parametrize("M", [96, 300])
-def test_tail_parts_past_the_edge(dev, M):
-    """Split tiles whose last rows and columns lie past the matrix (no partials are kept for
-    those blocks): a ragged M below and above one tile, N inside a tile's first 64 columns."""
-    N, K = 1064, 2560
+@pytest.mark.parametrize("M,N", [(96, 1064), (300, 1064), (289, 1032), (288, 1288), (512, 1280)])
+def test_tail_parts_past_the_edge(dev, M, N):
+    """Split tiles of the 256x256 core whose last rows and columns lie past the matrix (no partials
+    are kept for those blocks) and whole ones: a ragged M below and above one tile, on and off a
+    block of 32 rows, N inside a tile's first 64 columns. The one-pass LUT GEMMs and the dense
+    entries, each of which asks for the partials' workspace at these sizes."""
+    K = 2560
     idx, pal, x, W, (a, b) = _oracle_problem(M, N, K, seed=M, rank=16)
-    assert ops.query("plz_lut_linear_fwd_workspace", M, N, K) > 0
-    p, pl = _packed(idx, dev), pal.to(dev)
-    assert_close(f32(ops.lut_linear_fwd(x.to(dev), p, pl)), O.lut_linear_fwd(f32(x), W),
-                 what="fwd")
+    assert ops.query("plz_linear_fwd_dense_workspace", M, N, K) > 0
+    assert ops.query("plz_linear_bwd_x_dense_workspace", M, N, K) > 0
+    p, pl, xd = _packed(idx, dev), pal.to(dev), x.to(dev)
+    wd = ops.dequant(p, pl)
+    res = randn_bf16(M, N, seed=5).to(dev)
+    want = O.lut_linear_fwd(f32(x), W)
+    assert_close(f32(ops.lut_linear_fwd(xd, p, pl, staged=False)), want, what="fwd (LUT GEMM)")
+    y = ops.linear_fwd_dense(xd, wd)
+    assert_close(f32(y), want, what="dense fwd")
+    assert torch.equal(ops.linear_fwd_dense(xd, wd, residual=res), y + res)
     gy = randn_bf16(M, N, seed=4)
-    assert_close(f32(ops.lut_linear_bwd_x(gy.to(dev), p, pl)), O.grad_x(f32(gy), W),
-                 what="grad_x")
+    want = O.grad_x(f32(gy), W)
+    assert_close(f32(ops.lut_linear_bwd_x(gy.to(dev), p, pl, staged=False)), want,
+                 what="grad_x (LUT GEMM)")
+    assert_close(f32(ops.linear_bwd_x_dense(gy.to(dev), wd)), want, what="dense grad_x")
