@@ -3,7 +3,9 @@
 #undef NDEBUG
 #include <cassert>
 #include <cstdio>
+#include <set>
 
+#include "plz_attn_items.h"
 #include "plz_gemv_split.h"
 
 static long checks = 0;
@@ -41,7 +43,30 @@ static void check_gemv_split() {
   }
 }
 
+// Attention items: every (query block, batch, query head) once, the longest first, the kv head its
+// own; the heads of a pair on one XCD (id % 8) where the pairs divide by 8, and one query head per
+// kv head in batch-major order, as the dK/dV kernel's.
+static void check_attn_items() {
+  using namespace plz::attn;
+  for (int nqb : {1, 3, 4})
+    for (int B : {1, 2, 3, 8, 16})
+      for (const auto& heads : {std::pair<int, int>{1, 1}, {8, 8}, {6, 2}, {32, 8}, {16, 2}, {2, 1}}) {
+        const int Hq = heads.first, Hkv = heads.second, G = Hq / Hkv;
+        std::set<int> seen;
+        for (int id = 0; id < nqb * B * Hq; ++id) {
+          const QItem q = q_item(id, nqb, B, Hq, Hkv);
+          assert(q.qb == nqb - 1 - id / (B * Hq) && q.b >= 0 && q.b < B && q.h >= 0 && q.h < Hq);
+          assert(q.hk == q.h / G);
+          assert(seen.insert((q.qb * B + q.b) * Hq + q.h).second);
+          if (G == 1) assert(q.b * Hq + q.h == id % (B * Hq));
+          if (G > 1 && B * Hkv % 8 == 0) assert((q.b * Hkv + q.hk) / (B * Hkv / 8) == id % 8);
+          ++checks;
+        }
+      }
+}
+
 int main() {
+  check_attn_items();
   check_gemv_split();
   printf("launch rules: %ld checks passed\n", checks);
   return 0;
