@@ -1735,9 +1735,18 @@ constexpr int kDenseGroup = 4;
 // Up to 64 rows the forward runs the kernel of plz_skinny.hip: M = 17 / 48 / 64 in us against the
 // split 256-row tiles 2560 -> 4096 6.7 / 10.9 / 13.0 (24.0 / 34.7 / 34.8), 2560 -> 9728
 // 11.3 / 17.2 / 18.5 (27.8 / 37.8 / 37.8), 9728 -> 2560 17.5 / 32.6 / 41.0 (32.0 / 61.4 / 61.5). Its
-// time grows with M; at 128 rows 9728 -> 2560 is the slower one (80 against 65).
-static bool skinny_fwd_rows(int64_t M, int64_t K) {
-  return K > 0 && M <= sk::kMaxRows && M * K < ((int64_t)1 << 31);
+// time grows with M; at 128 rows 9728 -> 2560 is the slower one (80 against 65). Every workgroup
+// reads all of x: where N gives the split tiles few tiles, long reductions of many rows are theirs
+// (at M K = 1.05 / 1.24 / 1.64 million, N = 128: 68 / 78 / 102 us against 66 / 70 / 77; N 9728 at 1.43 /
+// 1.64 million 140 / 149 and 141 / 143; N 16384 at 4.2 million 411 and 516). And of W rows of 2 or 4
+// units of 128, which leave waves without work, in many rounds: 256 -> 65536 at M = 32 / 33 / 64
+// 12.5 / 16.4 / 16.6 and 13.3 (512: M = 48 / 64 19.2 / 22.0 and 20.0).
+static bool skinny_fwd_rows(int64_t M, int64_t N, int64_t K) {
+  if (K <= 0 || M > sk::kMaxRows || M * K >= ((int64_t)1 << 31)) return false;
+  const int64_t C = cu_count();
+  if (N > 128 * C) return M <= 16 + K / 16;
+  if (N >= 64 * C || (N >= 32 * C && M <= 32)) return true;
+  return M * K <= ((int64_t)(N >= 32 * C ? 12 : 9) << 17);
 }
 
 static size_t staged_w_bytes(int64_t N, int64_t K) {
@@ -1767,7 +1776,7 @@ static bool stage_w(Args& g, const int32_t* packed, const float* palette, int64_
 extern "C" {
 
 size_t plz_lut_linear_fwd_workspace(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0 || skinny_fwd_rows(M, K)) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || skinny_fwd_rows(M, N, K)) return 0;
   if (M >= kStagedRows) return staged_w_bytes(N, K) + tail_bytes(M, N, K);
   return tail_bytes(M, N, K);
 }
@@ -1787,7 +1796,7 @@ int plz_lut_linear_fwd(const uint16_t* x, const int32_t* packed, const float* pa
               "plz_lut_linear_fwd: x, packed and palette must be 16-byte aligned");
   PLZ_REQUIRE(rank == 0 || (lora_t && lora_b && a16(lora_t) && a16(lora_b)),
               "plz_lut_linear_fwd: rank > 0 needs 16-byte aligned lora_t and lora_b");
-  if (skinny_fwd_rows(M, K))
+  if (skinny_fwd_rows(M, N, K))
     return sk::fwd(x, packed, palette, bias, lora_t, lora_b, rank, y, M, N, K, cu_count(),
                    (hipStream_t)stream, "plz_lut_linear_fwd");
   Args g = {};

@@ -220,6 +220,18 @@ def test_lut_gemms_of_wide_outputs_stay_where_they_are_faster(lib, M, J, R, stag
         assert lib.plz_lut_linear_staged_pair(M, J, R) == staged
 
 
+@pytest.mark.parametrize("M,N,K,few_rows", [
+    (64, 2560, 9728, True), (64, 128, 16384, True), (64, 128, 25600, False),
+    (48, 1024, 49152, False), (16, 1024, 49152, True), (56, 9728, 25600, True),
+    (64, 9728, 49152, False), (32, 9728, 65536, True), (64, 16384, 65536, True), (65, 2560, 9728, False)])
+def test_long_reductions_of_few_tiles_are_split_tiles(lib, M, N, K, few_rows):
+    """The forward's kernel for few rows needs no workspace; the split 256-row tiles do (256 CUs)."""
+    if torch.cuda.is_available() and \
+            torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes for 256 CUs")
+    assert (lib.plz_lut_linear_fwd_workspace(M, N, K) == 0) == few_rows
+
+
 def test_attention_argument_errors(lib):
     """Shape, support and workspace checks of the attention entry points fail before any GPU
     work (pointer 16 stands for an aligned device pointer and is never dereferenced)."""

@@ -394,11 +394,12 @@ def test_gemv_split_launch_is_the_streaming_launch_bit_for_bit(dev, M, N, K):
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 64, 65])
 @pytest.mark.parametrize("N,K,rank,bias", [(8, 256, 0, True), (136, 768, 8, False),
                                            (1000, 2304, 40, True), (4104, 256, 32, False),
-                                           (8200, 512, 64, True)])
+                                           (8200, 512, 64, True), (128, 25600, 16, True),
+                                           (33000, 256, 8, False)])
 def test_lut_linear_fwd_few_rows(dev, M, N, K, rank, bias):
     """The forward's kernel for up to 64 rows (one to four 16-row blocks of W per workgroup, by N;
     one to four blocks of tokens; units of 128 k over eight waves; ranks past one 32-wide step)
-    and the first size past it."""
+    and the first size past it; a reduction and an output whose later Ms leave it for the tiles."""
     idx, pal, x, W, (a, b) = _oracle_problem(M, N, K, seed=M + N, rank=max(rank, 8))
     bv = randn_bf16(N, seed=3, std=0.1) if bias else None
     t = randn_bf16(M, rank, seed=5, std=0.1).to(dev) if rank else None
