@@ -18,6 +18,7 @@ from __future__ import annotations
 import math
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn as nn
 
 from . import fused_lut_linear_cuda as FL
@@ -162,10 +163,12 @@ class QwenLoRA(nn.Module):
 
 def _adds_in_epilogue(y_base, x, shape):
     """True where the GEMM kernel may read the base output itself: on x's device (a tensor of
-    another one is left to torch's add, which refuses it), dense, aligned bf16 of the very shape."""
+    another one is left to torch's add, which refuses it), dense, aligned bf16 of the very shape,
+    and without a forward-mode tangent, which torch's add carries on and the function does not."""
     return (y_base.is_cuda and y_base.device == x.device and y_base.dtype == torch.bfloat16
             and y_base.is_contiguous() and tuple(y_base.shape) == shape
-            and y_base.numel() > 0 and y_base.data_ptr() % 16 == 0)
+            and y_base.numel() > 0 and y_base.data_ptr() % 16 == 0
+            and fwAD.unpack_dual(y_base).tangent is None)
 
 
 class _LoRAFunction(torch.autograd.Function):

@@ -201,6 +201,27 @@ def test_lora_epilogue_reads_only_base_outputs_of_its_own_device():
     assert not _adds_in_epilogue(tensor(shape=(0, 8)), x, (0, 8))
 
 
+def test_forward_mode_tangent_of_the_base_output_is_left_to_the_add():
+    """A base output with a tangent (a plain base layer under forward-mode differentiation) is not
+    handed to the function, which has no forward-mode rule (a CPU tensor as the stand-in)."""
+    import torch.autograd.forward_ad as fwAD
+    from palettize_hip.qwen_model import _adds_in_epilogue
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+
+    base = torch.zeros(2, 8, dtype=torch.bfloat16).as_subclass(OnGpu)
+    x = torch.zeros(2, 16, dtype=torch.bfloat16)
+    aligned = base.data_ptr() % 16 == 0
+    assert _adds_in_epilogue(base, x, (2, 8)) == aligned
+    with fwAD.dual_level():
+        assert _adds_in_epilogue(base, x, (2, 8)) == aligned
+        dual = fwAD.make_dual(torch.zeros(2, 8, dtype=torch.bfloat16),
+                              torch.ones(2, 8, dtype=torch.bfloat16)).as_subclass(OnGpu)
+        assert fwAD.unpack_dual(dual).tangent is not None
+        assert not _adds_in_epilogue(dual, x, (2, 8))
+
+
 @pytest.mark.parametrize("M,J,R,staged", [
     # one LUT GEMM of M x J outputs over R at both sides of the rule (256 CUs)
     (48, 4096, 2560, 0), (128, 4096, 2560, 1), (1000, 4096, 2560, 1), (777, 9728, 2560, 0),
