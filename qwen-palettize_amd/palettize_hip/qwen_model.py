@@ -190,9 +190,13 @@ class _LoRAFunction(torch.autograd.Function):
     def backward(ctx, gy):
         from . import ops
         x, a_rk, b_nr, t = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        g_res = gy if need[4] else None
+        if not any(need[:3]):  # a frozen adapter on a base that trains
+            return None, None, None, None, g_res
         gy = gy.contiguous()
         gt = ops.lora_grad_t(gy, b_nr, ctx.scale)            # s * gy B   [M, r]
         # gt A^T
-        gx = ops.linear_bwd_x_dense(gt, a_rk, tiled=True) if ctx.needs_input_grad[0] else None
+        gx = ops.linear_bwd_x_dense(gt, a_rk, tiled=True) if need[0] else None
         ga, gb = ops.lora_weight_grads(x, gy, t, gt, 1.0, out_dtype=torch.bfloat16)
-        return gx, ga.t(), gb, None, gy if ctx.needs_input_grad[4] else None
+        return gx, ga.t(), gb, None, g_res

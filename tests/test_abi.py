@@ -201,6 +201,41 @@ def test_lora_epilogue_reads_only_base_outputs_of_its_own_device():
     assert not _adds_in_epilogue(tensor(shape=(0, 8)), x, (0, 8))
 
 
+def _lora_on_the_cpu(monkeypatch, ran):
+    """QwenLoRA's function with torch in the place of the kernels, which `ran` lists."""
+    from palettize_hip import ops
+
+    def op(name, f):
+        monkeypatch.setattr(ops, name, lambda *a, **k: ran.append(name) or f(*a, **k))
+
+    op("lora_project", lambda x, a, s: s * x @ a.t())
+    op("linear_fwd_dense",
+       lambda x, w, residual=None, tiled=False: x @ w.t() + (0 if residual is None else residual))
+    op("lora_grad_t", lambda gy, b, s: s * gy @ b)
+    op("linear_bwd_x_dense", lambda gt, a, tiled=False: gt @ a)
+    op("lora_weight_grads", lambda x, gy, t, gt, s, out_dtype=None: (gt.t() @ x, gy.t() @ t))
+
+
+def test_frozen_lora_runs_no_kernel_in_the_backward_of_its_base(monkeypatch):
+    """The base output's gradient passes through the function that adds it; without a gradient for
+    x, A or B nothing else is made."""
+    from palettize_hip.qwen_model import _LoRAFunction
+    ran = []
+    _lora_on_the_cpu(monkeypatch, ran)
+    g = torch.Generator().manual_seed(1)
+    x, A, B, base, gy = (torch.randn(*s, generator=g) for s in
+                         ((3, 8), (8, 2), (6, 2), (3, 6), (3, 6)))
+    base.requires_grad_(True)
+    y = _LoRAFunction.apply(x, A, B, 2.0, base)
+    assert torch.allclose(y, base + 2.0 * x @ A @ B.t())
+    ran.clear()
+    y.backward(gy)
+    assert torch.equal(base.grad, gy) and ran == []
+    A.requires_grad_(True)
+    _LoRAFunction.apply(x, A, B, 2.0, base).backward(gy)
+    assert torch.allclose(A.grad, 2.0 * x.t() @ (gy @ B), atol=1e-5)
+
+
 def test_forward_mode_tangent_of_the_base_output_is_left_to_the_add():
     """A base output with a tangent (a plain base layer under forward-mode differentiation) is not
     handed to the function, which has no forward-mode rule (a CPU tensor as the stand-in)."""
