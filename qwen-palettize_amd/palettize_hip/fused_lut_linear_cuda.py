@@ -337,11 +337,12 @@ def _noise_to_native(noise: Tensor, K: int, N: int, Kp: int) -> Tensor:
 
 def _soft_in_reference_layout(x, palette, logits, N, K, group_size):
     """True where the soft linear runs in the (K, N) order of its logits (plz_soft_ref_*): whole
-    8-element chunks along both dimensions, the palette in a type its kernels read. On
+    8-element chunks along both dimensions, K within a grid of 32-row blocks, the palette in a type
+    its kernels read. On
     2560 -> 4096 at 2048 rows that takes the two plane transposes (206 us each), the noise tensor
     and its reads out of a training pass. Other sizes go through the native layout, K padded."""
     return (x.is_cuda and logits.is_cuda and palette.is_cuda and x.dtype == torch.bfloat16
-            and x.dim() == 2 and x.shape[0] > 0 and N > 0 and K > 0 and K % 8 == 0
+            and x.dim() == 2 and x.shape[0] > 0 and N > 0 and 0 < K <= 32 * 65535 and K % 8 == 0
             and palette.dim() == 2 and palette.shape[1] == 4
             and palette.shape[0] >= _groups_used(N, group_size)
             and palette.dtype in (torch.bfloat16, torch.float16, torch.float32)

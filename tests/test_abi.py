@@ -201,6 +201,25 @@ def test_lora_epilogue_reads_only_base_outputs_of_its_own_device():
     assert not _adds_in_epilogue(tensor(shape=(0, 8)), x, (0, 8))
 
 
+@pytest.mark.parametrize("K,kept", [(8, True), (2560, True), (32 * 65535, True),
+                                    (32 * 65535 + 8, False), (12, False)])
+def test_soft_linear_keeps_to_the_reference_layout_where_its_kernels_take_it(lib, K, kept):
+    """What the (K, N)-order kernels refuse goes through the native layout (stand-ins for GPU
+    tensors: the rule looks at these properties only)."""
+    from types import SimpleNamespace
+    from palettize_hip import _lib as L, fused_lut_linear_cuda as FL
+
+    def tensor(shape, dtype=torch.bfloat16):
+        return SimpleNamespace(is_cuda=True, dtype=dtype, shape=shape, dim=lambda: len(shape),
+                               is_contiguous=lambda: True, data_ptr=lambda: 256)
+
+    x, pal, logits = tensor((2, K)), tensor((1, 4)), tensor((4, K, 8), torch.float16)
+    assert FL._soft_in_reference_layout(x, pal, logits, 8, K, 256) == kept
+    if not kept:  # and the kernels do refuse these: nothing is launched
+        assert lib.plz_soft_ref_build_w(256, L.PLZ_DT_FP16, 256, L.PLZ_DT_BF16, 256, 0, 1, 1.0,
+                                        L.PLZ_W_SOFT, 256, K, 8, None) != L.PLZ_OK
+
+
 def _lora_on_the_cpu(monkeypatch, ran):
     """QwenLoRA's function with torch in the place of the kernels, which `ran` lists."""
     from palettize_hip import ops
