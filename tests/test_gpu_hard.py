@@ -85,7 +85,9 @@ def _oracle_problem(M, N, K, seed, rank=0):
     (4097, 1032, 768, 8),
 ])
 def test_lut_linear_fwd(dev, M, N, K, rank):
-    """From 4096 rows the call dequantises W into its workspace and runs the dense GEMM."""
+    """The call's own route (from 65 rows here W dequantised and a dense GEMM on it, in the call's
+    workspace from 4096) and the one-pass one."""
+    assert ops.lut_linear_staged(M, N, K) == (M > 64)
     idx, pal, x, W, lora = _oracle_problem(M, N, K, seed=M + N + K, rank=rank)
     bias = randn_bf16(N, seed=5, std=0.1) if M % 2 else None
     args = {}
@@ -102,17 +104,19 @@ def test_lut_linear_fwd(dev, M, N, K, rank):
     if rank:
         want = want + O.lora_forward(f32(x), t_ref, f32(lora[1]), 1.0)
     assert_close(f32(y), want, what="y")
-    if M >= 4096:  # the one-pass LUT GEMM on the same problem
-        y1 = ops.lut_linear_fwd(x.to(dev), _packed(idx, dev), pal.to(dev),
-                                None if bias is None else bias.to(dev), staged=False, **args)
-        assert_close(f32(y1), want, what="y (LUT GEMM)")
+    # in one pass on the same problem
+    y1 = ops.lut_linear_fwd(x.to(dev), _packed(idx, dev), pal.to(dev),
+                            None if bias is None else bias.to(dev), staged=False, **args)
+    assert_close(f32(y1), want, what="y (one pass)")
 
 
 @pytest.mark.parametrize("M,N,K,rank", [(512, 2560, 2560, 16), (1, 256, 256, 0),
                                         (77, 1032, 768, 8), (256, 384, 1024, 32),
                                         (4096, 1032, 768, 8)])
 def test_lut_linear_bwd_x(dev, M, N, K, rank):
-    """From 4096 rows the call dequantises W into its workspace and runs the dense GEMM."""
+    """The call's own route (from 65 rows here W dequantised and a dense GEMM on it, in the call's
+    workspace from 4096) and the one-pass one."""
+    assert ops.lut_linear_staged(M, K, N) == (M > 64)
     idx, pal, _, W, lora = _oracle_problem(M, N, K, seed=3 * M + N, rank=rank)
     gy = randn_bf16(M, N, seed=9)
     args = {}
@@ -125,9 +129,9 @@ def test_lut_linear_bwd_x(dev, M, N, K, rank):
         want = want + f32(gt) @ f32(a)
     gx = ops.lut_linear_bwd_x(gy.to(dev), _packed(idx, dev), pal.to(dev), **args)
     assert_close(f32(gx), want, what="grad_x")
-    if M >= 4096:  # the one-pass LUT GEMM on the same problem
-        g1 = ops.lut_linear_bwd_x(gy.to(dev), _packed(idx, dev), pal.to(dev), staged=False, **args)
-        assert_close(f32(g1), want, what="grad_x (LUT GEMM)")
+    # in one pass on the same problem
+    g1 = ops.lut_linear_bwd_x(gy.to(dev), _packed(idx, dev), pal.to(dev), staged=False, **args)
+    assert_close(f32(g1), want, what="grad_x (one pass)")
 
 
 @pytest.mark.parametrize("M,N,K", [(512, 2560, 2560), (1, 256, 256), (77, 1032, 768),
@@ -389,6 +393,38 @@ def test_gemv_split_launch_is_the_streaming_launch_bit_for_bit(dev, M, N, K):
     assert torch.equal(split, streamed)
     assert_close(f32(split), O.lut_linear_fwd(f32(x), O.dequant(idx.numpy(), pal.numpy())),
                  what=f"split gemv M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("n", [7, 64, 65, 150])
+def test_gemv_split_launch_of_many_and_empty_linears(dev, M, n):
+    """A split launch finds its workgroups' linears in a table of up to 64 by a ballot, in a longer
+    one by a binary search, also past linears without rows (first, in a row, last): each linear's
+    outputs are those of its own launch, and of a streamed one."""
+    K, kinds = 512, []
+    for i, N in enumerate((8, 136)):
+        idx, pal = make_weight(N, K, seed=N)
+        kinds.append((_packed(idx, dev), pal.to(dev)))
+    empty = (torch.empty(0, K // 16, dtype=torch.int32, device=dev),
+             torch.empty(0, K // 256, 4, device=dev))
+    x = [randn_bf16(M, K, seed=s).to(dev) for s in range(3)]
+    items = []
+    for i in range(n):
+        w = empty if i in (0, 3, 4, n - 1) else kinds[0 if n > 100 or i % 5 else 1]
+        items.append((x[i % 3], *w))
+    got = ops.GemvGroup(items, layout="planes").run()
+    own = {}
+    for (xi, p, pl), y in zip(items, got):
+        assert tuple(y.shape) == (M, p.shape[0])
+        if p.shape[0]:
+            key = (xi.data_ptr(), p.data_ptr())
+            if key not in own:
+                own[key] = ops.GemvGroup([(xi, p, pl)], layout="planes").run()[0]
+            assert torch.equal(y, own[key])
+    idx2, pal2 = make_weight(128 * 300, 256, seed=1)
+    big = (randn_bf16(M, 256, seed=2).to(dev), _packed(idx2, dev), pal2.to(dev))
+    for y, z in zip(got, ops.GemvGroup(items + [big], layout="planes").run()):
+        assert torch.equal(y, z)
 
 
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 64, 65])

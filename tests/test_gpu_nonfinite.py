@@ -25,11 +25,14 @@ def _weight(N, K, seed, dev):
     return idx, ops.pack_indices(idx.to(dev)), pal.to(dev)
 
 
-@pytest.mark.parametrize("M,N,K,staged", [(300, 1032, 768, True), (4096, 2560, 2560, True),
-                                          (4096, 2560, 2560, False)])
+@pytest.mark.parametrize("M,N,K,staged", [(300, 1032, 768, True), (300, 1032, 768, False),
+                                          (4096, 2560, 2560, True), (4096, 2560, 2560, False),
+                                          (5, 136, 768, False), (17, 1032, 768, False),
+                                          (48, 4104, 512, False), (64, 8200, 256, False)])
 def test_forward_rows_of_a_nonfinite_input_go_nonfinite(dev, M, N, K, staged):
-    """staged: from 4096 rows W dequantised into the workspace and the dense GEMM; else the
-    one-pass LUT GEMM."""
+    """staged: W dequantised (from 4096 rows into the workspace) and a dense GEMM on it; else the
+    one-pass LUT GEMM, or up to 64 rows the kernel for few rows."""
+    assert ops.lut_linear_staged(M, N, K) >= staged
     _, p, pl = _weight(N, K, 1, dev)
     x = randn_bf16(M, K, seed=2).to(dev)
     clean = ops.lut_linear_fwd(x, p, pl, staged=staged)
@@ -69,15 +72,17 @@ def test_planes_gemv_tokens_of_a_nonfinite_input_go_nonfinite(dev, M):
     assert torch.equal(y[~bad], clean[~bad])
 
 
-@pytest.mark.parametrize("M", [512, 4096])  # the LUT GEMM; dequantised W + dense GEMM
-def test_grad_x_rows_of_a_nonfinite_gradient_go_nonfinite(dev, M):
+@pytest.mark.parametrize("staged", [True, False])  # dequantised W + dense GEMM; the LUT GEMM
+@pytest.mark.parametrize("M", [512, 4096])
+def test_grad_x_rows_of_a_nonfinite_gradient_go_nonfinite(dev, M, staged):
     N, K = 1024, 2560
+    assert ops.lut_linear_staged(M, K, N)
     _, p, pl = _weight(N, K, 3, dev)
     gy = randn_bf16(M, N, seed=4).to(dev)
-    clean = ops.lut_linear_bwd_x(gy, p, pl)
+    clean = ops.lut_linear_bwd_x(gy, p, pl, staged=staged)
     g2 = gy.clone()
     g2[17, 9] = NAN
-    gx = ops.lut_linear_bwd_x(g2, p, pl)
+    gx = ops.lut_linear_bwd_x(g2, p, pl, staged=staged)
     assert bool(torch.isnan(gx[17]).all())
     rows = torch.arange(M, device=dev) != 17
     assert torch.equal(gx[rows], clean[rows])
@@ -122,6 +127,42 @@ def test_soft_build_w_with_a_nan_logit(dev):
     mask = torch.ones(N, K, dtype=torch.bool, device=dev)
     mask[7, 33] = False
     assert torch.equal(w1[mask], w0[mask]) and torch.equal(s1[mask], s0[mask])
+
+
+@pytest.mark.parametrize("variant", ["cuda", "triton"])
+def test_soft_reference_layout_with_nonfinite_logits(dev, variant):
+    """The (K, N)-order build and backward: a NaN logit, and one of +inf (whose softmax is NaN),
+    make that weight's W_soft, its logits' gradients and its group's palette gradient non-finite;
+    the noisy hard pick keeps the first entry (comparisons with NaN are false). A logit of -inf is a
+    class of probability 0. Other weights do not move."""
+    K, N, GS, M = 264, 520, 256, 40
+    g = torch.Generator().manual_seed(13)
+    logits = torch.randn(4, K, N, generator=g).to(torch.float16).to(dev)
+    pal = (torch.randn(3, 4, generator=g) * 0.02).to(torch.bfloat16).to(dev)
+    x, gy = randn_bf16(M, K, seed=14).to(dev), randn_bf16(M, N, seed=15).to(dev)
+    bad = [(2, 33, 300, NAN), (0, 260, 301, INF), (3, 5, 7, -INF)]
+    lb = logits.clone()
+    for c, k, n, v in bad:
+        lb[c, k, n] = v
+    moved = torch.zeros(K, N, dtype=torch.bool, device=dev)
+    for _, k, n, _ in bad:
+        moved[k, n] = True
+    build = lambda lg, mode: ops.soft_ref_build_w(lg, pal, GS, 9, 0.5, mode, variant)  # noqa: E731
+    soft, clean = build(lb, PLZ_W_SOFT), build(logits, PLZ_W_SOFT)
+    assert not bool(torch.isfinite(soft[[33, 260], [300, 301]]).any())
+    assert bool(torch.isfinite(soft[5, 7]))
+    assert torch.equal(soft[~moved], clean[~moved])
+    hard = build(lb, PLZ_W_HARD_NOISY)
+    assert torch.equal(hard[[33, 260], [300, 301]], pal[1, 0].expand(2))
+    assert float(hard[5, 7]) in pal[0, :3].float().tolist()
+    assert torch.equal(hard[~moved], build(logits, PLZ_W_HARD_NOISY)[~moved])
+    gl0, gp0 = ops.soft_ref_bwd(x, gy, logits, pal, GS, 9, 0.5, variant)
+    gl, gp = ops.soft_ref_bwd(x, gy, lb, pal, GS, 9, 0.5, variant)
+    assert not bool(torch.isfinite(gl[:, [33, 260], [300, 301]]).any())
+    assert float(gl[3, 5, 7]) == 0.0 and bool(torch.isfinite(gl[:, 5, 7]).all())
+    assert torch.equal(gl[:, ~moved], gl0[:, ~moved])
+    assert not bool(torch.isfinite(gp[1]).any()) and bool(torch.isfinite(gp[0]).all())
+    assert torch.equal(gp[2], gp0[2])
 
 
 def test_distillation_loss_of_a_nan_student_is_nan(dev):
