@@ -344,21 +344,6 @@ __device__ __forceinline__ u32x4 add_residual8(u32x4 v, const uint16_t* r) {
   return o;
 }
 
-// 8 stored bf16 values of grad_h at (i, j) through the SwiGLU backward: its gate and up gradients
-// for the [gate | up] pre-activations pre [I, 2J] (row stride ld_sw) go to columns j and J + j of
-// the [I, 2J] output (row stride ldc)
-__device__ __forceinline__ void store_swiglu_bwd8(u32x4 v, const uint16_t* sw_pre, int64_t ld_sw,
-                                                  uint16_t* C, int64_t ldc, int64_t J, int64_t i,
-                                                  int64_t j) {
-  const uint16_t* pre = sw_pre + i * ld_sw + j;
-  uint4 gg, gu;
-  swiglu_bwd8(*reinterpret_cast<const uint4*>(pre), *reinterpret_cast<const uint4*>(pre + J),
-              make_uint4(v[0], v[1], v[2], v[3]), gg, gu);
-  const u32x4 a = {gg.x, gg.y, gg.z, gg.w}, b = {gu.x, gu.y, gu.z, gu.w};
-  __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(C + i * ldc + j));
-  __builtin_nontemporal_store(b, reinterpret_cast<u32x4*>(C + i * ldc + J + j));
-}
-
 // ---- work-item map and launch planning (shared by the kernels and a host-side check) -------
 // A launch has tiles_i x tiles_j output tiles and gridDim.z reduction splits; a tail-split
 // launch (bf16 epilogue, tail_split > 1) runs its first tail_first tiles whole and each later

@@ -721,6 +721,19 @@ __device__ __forceinline__ void stage_tile_bf16(const Args& g, const f32x16 (&ac
       }
   __syncthreads();
 }
+// 8 stored bf16 values of grad_h at (i, j) through the SwiGLU backward (g.sw_pre set): its gate
+// and up gradients go to columns j and J + j of the [I, 2J] output
+__device__ __forceinline__ void store_swiglu_bwd8(const Args& g, u32x4 v, uint16_t* C, int64_t i,
+                                                  int64_t j) {
+  const uint16_t* pre = g.sw_pre + i * g.ld_sw + j;
+  uint4 gg, gu;
+  swiglu_bwd8(*reinterpret_cast<const uint4*>(pre), *reinterpret_cast<const uint4*>(pre + g.J),
+              make_uint4(v[0], v[1], v[2], v[3]), gg, gu);
+  const u32x4 a = {gg.x, gg.y, gg.z, gg.w}, b = {gu.x, gu.y, gu.z, gu.w};
+  __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(C + i * g.ldc + j));
+  __builtin_nontemporal_store(b, reinterpret_cast<u32x4*>(C + i * g.ldc + g.J + j));
+}
+
 __device__ __forceinline__ void store_tile_bf16(const Args& g, const f32x16 (&acc)[WT_I][WT_J],
                                                 lds_u8* st, int64_t i0, int64_t j0, int wi,
                                                 int wj, int lane) {
@@ -737,7 +750,7 @@ __device__ __forceinline__ void store_tile_bf16(const Args& g, const f32x16 (&ac
       // streaming store: the output is not read again by this launch, so it should not take
       // cache lines from the operands the other workgroups are still reading
       if (g.sw_pre)
-        store_swiglu_bwd8(v, g.sw_pre, g.ld_sw, C, g.ldc, g.J, i, j);
+        store_swiglu_bwd8(g, v, C, i, j);
       else
         __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(C + i * g.ldc + j));
     }
@@ -1368,7 +1381,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void tail_reduce_kernel(const Args g)
       u32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(st + row * EPI_RS + c8 * 2);
       if (g.res) v = add_residual8(v, g.res + i * g.ldres + j);
       if (g.sw_pre)
-        store_swiglu_bwd8(v, g.sw_pre, g.ld_sw, C, g.ldc, g.J, i, j);
+        store_swiglu_bwd8(g, v, C, i, j);
       else
         __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(C + i * g.ldc + j));
     }
