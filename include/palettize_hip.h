@@ -180,9 +180,22 @@ int plz_linear_fwd_dense_swiglu(const uint16_t* x, const uint16_t* w_gate_up, ui
 int plz_linear_fwd_dense_swiglu_cat(const uint16_t* x, const uint16_t* w, const uint16_t* lora_t,
                                     const uint16_t* lora_b, int rank, uint16_t* y, uint16_t* h,
                                     int64_t M, int64_t F, int64_t K, void* stream);
-/* How a LUT GEMM of rows x outputs over a reduction (forward M, N, K; grad_x M, K, N) is fastest:
- * 0 in one pass (plz_lut_linear_fwd / _bwd_x); 1 plz_dequant and a tiled GEMM below on the bf16 W;
- * 2 so too, which those entries do themselves in the workspace that their queries ask for. */
+/* plz_lut_linear_fwd and plz_lut_linear_bwd_x on the schedule that is the faster one for the shape:
+ * where their workspace holds what the queries ask for, that may be W dequantised into it and a GEMM
+ * on 128x128 tiles on that W (sums over the reduction in another order), with fewer than 4096 rows
+ * too. With less, or elsewhere, as the entries without _tiled. */
+size_t plz_lut_linear_fwd_tiled_workspace(int64_t M, int64_t N, int64_t K);
+int plz_lut_linear_fwd_tiled(const uint16_t* x, const int32_t* packed, const float* palette,
+                             const uint16_t* bias, const uint16_t* lora_t, const uint16_t* lora_b,
+                             int rank, uint16_t* y, void* workspace, size_t workspace_bytes,
+                             int64_t M, int64_t N, int64_t K, void* stream);
+size_t plz_lut_linear_bwd_x_tiled_workspace(int64_t M, int64_t N, int64_t K);
+int plz_lut_linear_bwd_x_tiled(const uint16_t* grad_y, const int32_t* packed, const float* palette,
+                               const uint16_t* lora_gt, const uint16_t* lora_a, int rank,
+                               uint16_t* grad_x, void* workspace, size_t workspace_bytes, int64_t M,
+                               int64_t N, int64_t K, void* stream);
+/* How these run a LUT GEMM of rows x outputs over a reduction (forward M, N, K; grad_x M, K, N):
+ * 0 in one pass; 1 dequantised, 128x128 tiles; 2 (from 4096 rows) dequantised, either tiles. */
 int plz_lut_linear_staged(int64_t rows, int64_t outputs, int64_t reduction);
 /* The same for a forward whose bf16 W the grad_x of the same pass uses again. */
 int plz_lut_linear_staged_pair(int64_t M, int64_t N, int64_t K);

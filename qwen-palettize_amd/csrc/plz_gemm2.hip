@@ -1722,11 +1722,17 @@ constexpr int64_t kStagedRows = 4096;
 // then runs on the 128x128 core and the models say so. In us, LUT -> dequantise + dense: forward
 // 2560 -> 4096 at M = 128 / 1000 37 -> 26 / 53 -> 39, 9728 -> 2560 at M = 128 65 -> 36;
 // 777 x 2560 -> 9728 stays (67 against 71). The skinny forward's rows stay with it.
-static bool staged_rows(int64_t I, int64_t J, int64_t R) {
+static bool staged_rows(int64_t I, int64_t J, int64_t R, int* z = nullptr) {
+  if (I <= sk::kMaxRows) return false;
   double us;
-  return I > sk::kMaxRows && dense_splits(I, J, R, &us) > 0 &&
-         us + 2.9 + 0.385e-6 * (double)J * (double)R < 0.97 * core256_us(I, J, R, 1.55);
+  const int splits = dense_splits(I, J, R, &us);
+  if (z) *z = splits;
+  return splits > 0 && us + 2.9 + 0.385e-6 * (double)J * (double)R < 0.97 * core256_us(I, J, R, 1.55);
 }
+// A LUT GEMM shorter than the host takes to issue one (17 us through the binding, 19 with the
+// second launch) has nothing to gain: 256 -> 256, 4096 and 9728 and 512 -> 264 at M = 65 to 4095 17.1 to
+// 18.4 us a call in one pass and 18.6 to 20.2 staged.
+constexpr double kCallUs = 18.5;
 // ... for one GEMM by itself. Where W is wide (J > 3 R) the LUT core's few row tiles spread over many
 // columns, while the dense core reads a freshly written W from beyond the L2s, which costs more
 // than the models say once a CU holds two workgroups of it (short prefetch) or W is large: LUT
@@ -1734,8 +1740,8 @@ static bool staged_rows(int64_t I, int64_t J, int64_t R) {
 // 9728 at M = 128 / 256 / 640 28.7 / 28.6 / 28.5 and 28.4 / 24.9 / 34.6; 2560 -> 9728 at M = 128 /
 // 200 / 512 42.3 / 42.3 / 49.1 and 35.5 / 45.2 / 51.7. From 769 rows (2048 of 1024 -> 9728: 64.5 and
 // 56.2) and for 1280 -> 4864 (M = 640: 25.0 and 18.8) the models hold.
-static bool staged_alone(int64_t I, int64_t J, int64_t R) {
-  if (!staged_rows(I, J, R)) return false;
+static bool staged_alone(int64_t I, int64_t J, int64_t R, int* z = nullptr) {
+  if (core256_us(I, J, R, 1.55) < kCallUs || !staged_rows(I, J, R, z)) return false;
   if (J <= 3 * R || I <= 128 || I > 768) return true;
   const int64_t tiles = ((I + 127) / 128) * ((J + 127) / 128);  // of the 128x128 core
   return tiles <= cu_count() && (I > 256 || J * R < ((int64_t)1 << 24));
@@ -1786,6 +1792,36 @@ static bool stage_w(Args& g, const int32_t* packed, const float* palette, int64_
   return true;
 }
 
+// The *_tiled entries, where that is the faster way: W dequantised into the head of the workspace
+// and the 128x128 core on it, its partials behind W. One call for both launches: as two calls of
+// the binding small sizes waited for the host (1024 -> 1024 at M = 65 to 256 26.4 to 27.6 us a call,
+// 24.6 in one pass, 19.5 so).
+static size_t lut_mid_bytes(int64_t I, int64_t J, int64_t R, int* splits = nullptr) {
+  int z = 0;
+  if (I >= kStagedRows) z = dense_splits(I, J, R);
+  else if (!staged_alone(I, J, R, &z)) z = 0;
+  if (splits) *splits = z;
+  return z > 0 ? staged_w_bytes(J, R) + mid::workspace(I, J, z) : 0;
+}
+// Returns false (nothing launched) where the call is not to run so; else *rc holds its status. m
+// has the epilogue's fields.
+static bool lut_mid(mid::Args m, bool b_col, const int32_t* packed, const float* palette, int64_t N,
+                    int64_t K, void* workspace, size_t workspace_bytes, const char* what,
+                    void* stream, int* rc) {
+  if (!workspace || !a16(workspace)) return false;
+  int z;
+  const size_t need = lut_mid_bytes(m.I, m.J, m.R, &z);
+  if (need == 0 || workspace_bytes < need) return false;
+  uint16_t* w = reinterpret_cast<uint16_t*>(workspace);
+  *rc = plz_dequant(packed, palette, w, N, K, stream);
+  if (*rc != PLZ_OK) return true;
+  m.b = w; m.ldb = K;
+  *rc = mid::launch(m, b_col, z, cu_count(),
+                    static_cast<uint8_t*>(workspace) + staged_w_bytes(N, K), (hipStream_t)stream,
+                    what);
+  return true;
+}
+
 extern "C" {
 
 size_t plz_lut_linear_fwd_workspace(int64_t M, int64_t N, int64_t K) {
@@ -1794,40 +1830,60 @@ size_t plz_lut_linear_fwd_workspace(int64_t M, int64_t N, int64_t K) {
   return tail_bytes(M, N, K);
 }
 
-int plz_lut_linear_fwd(const uint16_t* x, const int32_t* packed, const float* palette,
-                       const uint16_t* bias, const uint16_t* lora_t, const uint16_t* lora_b,
-                       int rank, uint16_t* y, void* workspace, size_t workspace_bytes, int64_t M,
-                       int64_t N, int64_t K, void* stream) {
-  PLZ_REQUIRE(M >= 0 && N >= 0 && K >= 0, "plz_lut_linear_fwd: negative shape");
-  PLZ_REQUIRE(K % 256 == 0, "plz_lut_linear_fwd: K (%lld) must be a multiple of 256", (long long)K);
-  PLZ_REQUIRE(N % 8 == 0, "plz_lut_linear_fwd: N (%lld) must be a multiple of 8", (long long)N);
+static int lut_linear_fwd(const uint16_t* x, const int32_t* packed, const float* palette,
+                          const uint16_t* bias, const uint16_t* lora_t, const uint16_t* lora_b,
+                          int rank, uint16_t* y, void* workspace, size_t workspace_bytes, int64_t M,
+                          int64_t N, int64_t K, void* stream, const char* what, bool tiled) {
+  PLZ_REQUIRE(M >= 0 && N >= 0 && K >= 0, "%s: negative shape", what);
+  PLZ_REQUIRE(K % 256 == 0, "%s: K (%lld) must be a multiple of 256", what, (long long)K);
+  PLZ_REQUIRE(N % 8 == 0, "%s: N (%lld) must be a multiple of 8", what, (long long)N);
   PLZ_REQUIRE(rank >= 0 && rank <= BK && rank % 8 == 0,
-              "plz_lut_linear_fwd: rank (%d) must be a multiple of 8 in [0, 64]", rank);
+              "%s: rank (%d) must be a multiple of 8 in [0, 64]", what, rank);
   if (M == 0 || N == 0) return PLZ_OK;
-  PLZ_REQUIRE(x && packed && palette && y, "plz_lut_linear_fwd: null pointer");
+  PLZ_REQUIRE(x && packed && palette && y, "%s: null pointer", what);
   PLZ_REQUIRE(a16(x) && a16(palette) && a16(packed),
-              "plz_lut_linear_fwd: x, packed and palette must be 16-byte aligned");
+              "%s: x, packed and palette must be 16-byte aligned", what);
   PLZ_REQUIRE(rank == 0 || (lora_t && lora_b && a16(lora_t) && a16(lora_b)),
-              "plz_lut_linear_fwd: rank > 0 needs 16-byte aligned lora_t and lora_b");
+              "%s: rank > 0 needs 16-byte aligned lora_t and lora_b", what);
   if (skinny_fwd_rows(M, N, K))
     return sk::fwd(x, packed, palette, bias, lora_t, lora_b, rank, y, M, N, K, cu_count(),
-                   (hipStream_t)stream, "plz_lut_linear_fwd");
+                   (hipStream_t)stream, what);
+  int rc = PLZ_OK;
+  if (tiled) {
+    const mid::Args m = {x, K, nullptr, 0, M, N, K, lora_t, lora_b, rank, y, N, bias, nullptr, 0};
+    if (lut_mid(m, false, packed, palette, N, K, workspace, workspace_bytes, what, stream, &rc))
+      return rc;
+  }
   Args g = {};
   g.a = x; g.lda = K;
   g.I = M; g.J = N; g.R = K;
   g.a2 = lora_t; g.b2 = lora_b; g.R2 = rank;
   g.c = y; g.ldc = N; g.bias = bias; g.alpha = 1.f;
-  int rc = PLZ_OK;
-  if (stage_w(g, packed, palette, N, K, workspace, workspace_bytes, "plz_lut_linear_fwd", stream,
-              &rc)) {
+  if (stage_w(g, packed, palette, N, K, workspace, workspace_bytes, what, stream, &rc)) {
     if (rc != PLZ_OK) return rc;  // B(j=n, r=k) = w[n, k]   (Row tile)
-    return launch<OP_ROW, OP_ROW, EPI_BF16>(g, 1, (hipStream_t)stream, "plz_lut_linear_fwd");
+    return launch<OP_ROW, OP_ROW, EPI_BF16>(g, 1, (hipStream_t)stream, what);
   }
   g.packed = packed; g.pal = palette; g.Nw = N; g.Kw = K;
   g.group = 1;
-  rc = set_tail(g, workspace, workspace_bytes, "plz_lut_linear_fwd");
+  rc = set_tail(g, workspace, workspace_bytes, what);
   if (rc != PLZ_OK) return rc;
-  return launch<OP_ROW, OP_LUT_REG, EPI_BF16>(g, 1, (hipStream_t)stream, "plz_lut_linear_fwd");
+  return launch<OP_ROW, OP_LUT_REG, EPI_BF16>(g, 1, (hipStream_t)stream, what);
+}
+
+int plz_lut_linear_fwd(const uint16_t* x, const int32_t* packed, const float* palette,
+                       const uint16_t* bias, const uint16_t* lora_t, const uint16_t* lora_b,
+                       int rank, uint16_t* y, void* workspace, size_t workspace_bytes, int64_t M,
+                       int64_t N, int64_t K, void* stream) {
+  return lut_linear_fwd(x, packed, palette, bias, lora_t, lora_b, rank, y, workspace,
+                        workspace_bytes, M, N, K, stream, "plz_lut_linear_fwd", false);
+}
+
+int plz_lut_linear_fwd_tiled(const uint16_t* x, const int32_t* packed, const float* palette,
+                             const uint16_t* bias, const uint16_t* lora_t, const uint16_t* lora_b,
+                             int rank, uint16_t* y, void* workspace, size_t workspace_bytes,
+                             int64_t M, int64_t N, int64_t K, void* stream) {
+  return lut_linear_fwd(x, packed, palette, bias, lora_t, lora_b, rank, y, workspace,
+                        workspace_bytes, M, N, K, stream, "plz_lut_linear_fwd_tiled", true);
 }
 
 size_t plz_lut_linear_bwd_x_workspace(int64_t M, int64_t N, int64_t K) {
@@ -1836,38 +1892,68 @@ size_t plz_lut_linear_bwd_x_workspace(int64_t M, int64_t N, int64_t K) {
   return tail_bytes(M, K, N);
 }
 
-int plz_lut_linear_bwd_x(const uint16_t* grad_y, const int32_t* packed, const float* palette,
-                         const uint16_t* lora_gt, const uint16_t* lora_a, int rank,
-                         uint16_t* grad_x, void* workspace, size_t workspace_bytes, int64_t M,
-                         int64_t N, int64_t K, void* stream) {
-  PLZ_REQUIRE(M >= 0 && N >= 0 && K >= 0, "plz_lut_linear_bwd_x: negative shape");
-  PLZ_REQUIRE(K % 256 == 0, "plz_lut_linear_bwd_x: K (%lld) must be a multiple of 256",
-              (long long)K);
-  PLZ_REQUIRE(N % 8 == 0, "plz_lut_linear_bwd_x: N (%lld) must be a multiple of 8", (long long)N);
+static int lut_linear_bwd_x(const uint16_t* grad_y, const int32_t* packed, const float* palette,
+                            const uint16_t* lora_gt, const uint16_t* lora_a, int rank,
+                            uint16_t* grad_x, void* workspace, size_t workspace_bytes, int64_t M,
+                            int64_t N, int64_t K, void* stream, const char* what, bool tiled) {
+  PLZ_REQUIRE(M >= 0 && N >= 0 && K >= 0, "%s: negative shape", what);
+  PLZ_REQUIRE(K % 256 == 0, "%s: K (%lld) must be a multiple of 256", what, (long long)K);
+  PLZ_REQUIRE(N % 8 == 0, "%s: N (%lld) must be a multiple of 8", what, (long long)N);
   PLZ_REQUIRE(rank >= 0 && rank <= BK && rank % 8 == 0,
-              "plz_lut_linear_bwd_x: rank (%d) must be a multiple of 8 in [0, 64]", rank);
+              "%s: rank (%d) must be a multiple of 8 in [0, 64]", what, rank);
   if (M == 0 || K == 0) return PLZ_OK;
-  PLZ_REQUIRE(grad_y && packed && palette && grad_x, "plz_lut_linear_bwd_x: null pointer");
+  PLZ_REQUIRE(grad_y && packed && palette && grad_x, "%s: null pointer", what);
   PLZ_REQUIRE(a16(grad_y) && a16(palette) && a16(packed),
-              "plz_lut_linear_bwd_x: grad_y, packed and palette must be 16-byte aligned");
+              "%s: grad_y, packed and palette must be 16-byte aligned", what);
   PLZ_REQUIRE(rank == 0 || (lora_gt && lora_a && a16(lora_gt) && a16(lora_a)),
-              "plz_lut_linear_bwd_x: rank > 0 needs 16-byte aligned lora_gt and lora_a");
+              "%s: rank > 0 needs 16-byte aligned lora_gt and lora_a", what);
+  int rc = PLZ_OK;
+  if (tiled) {
+    const mid::Args m = {grad_y, N, nullptr, 0, M, K, N, lora_gt, lora_a, rank, grad_x, K, nullptr,
+                         nullptr, 0};
+    if (lut_mid(m, true, packed, palette, N, K, workspace, workspace_bytes, what, stream, &rc))
+      return rc;
+  }
   Args g = {};
   g.a = grad_y; g.lda = N;
   g.I = M; g.J = K; g.R = N;
   g.a2 = lora_gt; g.b2 = lora_a; g.R2 = rank;
   g.c = grad_x; g.ldc = K; g.alpha = 1.f;
-  int rc = PLZ_OK;
-  if (stage_w(g, packed, palette, N, K, workspace, workspace_bytes, "plz_lut_linear_bwd_x",
-              stream, &rc)) {
+  if (stage_w(g, packed, palette, N, K, workspace, workspace_bytes, what, stream, &rc)) {
     if (rc != PLZ_OK) return rc;  // B(j=k, r=n) = w[n, k]   (Col tile)
-    return launch<OP_ROW, OP_COL, EPI_BF16>(g, 1, (hipStream_t)stream, "plz_lut_linear_bwd_x");
+    return launch<OP_ROW, OP_COL, EPI_BF16>(g, 1, (hipStream_t)stream, what);
   }
   g.packed = packed; g.pal = palette; g.Nw = N; g.Kw = K;
   g.group = 1;
-  rc = set_tail(g, workspace, workspace_bytes, "plz_lut_linear_bwd_x");
+  rc = set_tail(g, workspace, workspace_bytes, what);
   if (rc != PLZ_OK) return rc;
-  return launch<OP_ROW, OP_LUT_COL, EPI_BF16>(g, 1, (hipStream_t)stream, "plz_lut_linear_bwd_x");
+  return launch<OP_ROW, OP_LUT_COL, EPI_BF16>(g, 1, (hipStream_t)stream, what);
+}
+
+int plz_lut_linear_bwd_x(const uint16_t* grad_y, const int32_t* packed, const float* palette,
+                         const uint16_t* lora_gt, const uint16_t* lora_a, int rank,
+                         uint16_t* grad_x, void* workspace, size_t workspace_bytes, int64_t M,
+                         int64_t N, int64_t K, void* stream) {
+  return lut_linear_bwd_x(grad_y, packed, palette, lora_gt, lora_a, rank, grad_x, workspace,
+                          workspace_bytes, M, N, K, stream, "plz_lut_linear_bwd_x", false);
+}
+
+int plz_lut_linear_bwd_x_tiled(const uint16_t* grad_y, const int32_t* packed, const float* palette,
+                               const uint16_t* lora_gt, const uint16_t* lora_a, int rank,
+                               uint16_t* grad_x, void* workspace, size_t workspace_bytes, int64_t M,
+                               int64_t N, int64_t K, void* stream) {
+  return lut_linear_bwd_x(grad_y, packed, palette, lora_gt, lora_a, rank, grad_x, workspace,
+                          workspace_bytes, M, N, K, stream, "plz_lut_linear_bwd_x_tiled", true);
+}
+
+size_t plz_lut_linear_fwd_tiled_workspace(int64_t M, int64_t N, int64_t K) {
+  const size_t m = M > 0 && N > 0 && K > 0 ? lut_mid_bytes(M, N, K) : 0;
+  return m > 0 ? m : plz_lut_linear_fwd_workspace(M, N, K);
+}
+
+size_t plz_lut_linear_bwd_x_tiled_workspace(int64_t M, int64_t N, int64_t K) {
+  const size_t m = M > 0 && N > 0 && K > 0 ? lut_mid_bytes(M, K, N) : 0;
+  return m > 0 ? m : plz_lut_linear_bwd_x_workspace(M, N, K);
 }
 
 size_t plz_lut_linear_bwd_palette_workspace(int64_t M, int64_t N, int64_t K) {

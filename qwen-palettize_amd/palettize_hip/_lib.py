@@ -81,6 +81,10 @@ SIGNATURES: dict[str, tuple] = {
     "plz_linear_fwd_dense_workspace": (sz, [i64, i64, i64]),
     "plz_linear_fwd_dense_swiglu": (i32, [p, p, p, i64, i64, i64, p]),
     "plz_linear_fwd_dense_swiglu_cat": (i32, [p, p, p, p, i32, p, p, i64, i64, i64, p]),
+    "plz_lut_linear_fwd_tiled": (i32, [p, p, p, p, p, p, i32, p, p, sz, i64, i64, i64, p]),
+    "plz_lut_linear_fwd_tiled_workspace": (sz, [i64, i64, i64]),
+    "plz_lut_linear_bwd_x_tiled": (i32, [p, p, p, p, p, i32, p, p, sz, i64, i64, i64, p]),
+    "plz_lut_linear_bwd_x_tiled_workspace": (sz, [i64, i64, i64]),
     "plz_lut_linear_staged": (i32, [i64, i64, i64]),
     "plz_lut_linear_staged_pair": (i32, [i64, i64, i64]),
     "plz_linear_tiled_workspace": (sz, [i64, i64, i64]),

@@ -26,10 +26,10 @@ def _c(t):
 
 
 class LUTLinearFunction(torch.autograd.Function):
-    """Where the forward dequantises W and runs a dense GEMM on it (ops.lut_linear_staged) and x
-    needs a gradient, the bf16 W is kept for the backward's grad_x instead of being dequantised a
-    second time (N*K*2 bytes held from forward to backward); without a gradient for x nothing
-    reads it, and it is dropped after the GEMM."""
+    """Where the forward runs a dense GEMM on a dequantised W (ops.lut_linear_staged) and x needs a
+    gradient, the bf16 W is kept for the backward's grad_x instead of being dequantised a second
+    time (N*K*2 bytes held from forward to backward); without a gradient for x it lives in the
+    call's workspace only."""
 
     @staticmethod
     def forward(ctx, x, packed, palette, bias, lora_a, lora_b, lora_scale):
@@ -37,12 +37,10 @@ class LUTLinearFunction(torch.autograd.Function):
         lora_a, lora_b = _c(lora_a), _c(lora_b)
         t = ops.lora_project(x, lora_a, lora_scale) if lora_a is not None else None
         w = None
-        if ops.lut_linear_staged(x.shape[0], packed.shape[0], x.shape[1],
-                                 grad_x=ctx.needs_input_grad[0]):
+        if ctx.needs_input_grad[0] and ops.lut_linear_staged(x.shape[0], packed.shape[0],
+                                                             x.shape[1], grad_x=True):
             w = ops.dequant(packed, palette)
             y = ops.linear_fwd_dense(x, w, bias, t, lora_b, tiled=True)
-            if not ctx.needs_input_grad[0]:
-                w = None
         else:
             y = ops.lut_linear_fwd(x, packed, palette, bias, t, lora_b)
         ctx.save_for_backward(x, packed, palette, lora_a, lora_b, t, w)

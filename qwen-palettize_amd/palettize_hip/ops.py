@@ -160,9 +160,9 @@ def lut_linear_staged(M: int, N: int, K: int, grad_x: bool = False) -> bool:
 def lut_linear_fwd(x, packed, palette, bias=None, lora_t=None, lora_b=None, staged=True):
     """y = x W^T (+ bias) (+ lora_t lora_b^T).
 
-    staged: dequantise W and run a dense GEMM on it where that is faster (lut_linear_staged; from
-    4096 rows inside the call, in the workspace that its query asks for); False keeps the
-    one-pass LUT GEMM (workspace for its tail partials only)."""
+    staged: W dequantised into the workspace and a dense GEMM on it where that is faster
+    (lut_linear_staged); False keeps the one-pass LUT GEMM (workspace for its tail partials
+    only)."""
     N, K = _wshape(packed, palette)
     _need(x, "x", torch.bfloat16, 2)
     M = x.shape[0]
@@ -170,12 +170,10 @@ def lut_linear_fwd(x, packed, palette, bias=None, lora_t=None, lora_b=None, stag
         raise ValueError(f"x has {x.shape[1]} columns, W has K={K}")
     _bias(bias, N)
     rank = _lora_pair(lora_t, lora_b, "lora_t", "lora_b", M, N)
-    if staged and query("plz_lut_linear_staged", M, N, K) == 1:
-        return linear_fwd_dense(x, dequant(packed, palette), bias, lora_t, lora_b, tiled=True)
     y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    q = "plz_lut_linear_fwd_workspace" if staged else "plz_linear_fwd_dense_workspace"
+    q = "plz_lut_linear_fwd_tiled_workspace" if staged else "plz_linear_fwd_dense_workspace"
     ws = _opt_workspace(query(q, M, N, K), x.device)
-    call("plz_lut_linear_fwd", _ptr(x), _ptr(packed), _ptr(palette), _ptr(bias), _ptr(lora_t),
+    call("plz_lut_linear_fwd_tiled" if staged else "plz_lut_linear_fwd", _ptr(x), _ptr(packed), _ptr(palette), _ptr(bias), _ptr(lora_t),
          _ptr(lora_b), rank, _ptr(y), _ptr(ws), _numel(ws), M, N, K, _stream(x))
     return y
 
@@ -183,9 +181,9 @@ def lut_linear_fwd(x, packed, palette, bias=None, lora_t=None, lora_b=None, stag
 def lut_linear_bwd_x(grad_y, packed, palette, lora_gt=None, lora_a=None, staged=True):
     """grad_x = grad_y W (+ lora_gt lora_a).
 
-    staged: dequantise W and run a dense GEMM on it where that is faster (lut_linear_staged; from
-    4096 rows inside the call, in the workspace that its query asks for); False keeps the
-    one-pass LUT GEMM (workspace for its tail partials only)."""
+    staged: W dequantised into the workspace and a dense GEMM on it where that is faster
+    (lut_linear_staged); False keeps the one-pass LUT GEMM (workspace for its tail partials
+    only)."""
     N, K = _wshape(packed, palette)
     _need(grad_y, "grad_y", torch.bfloat16, 2)
     M = grad_y.shape[0]
@@ -200,12 +198,10 @@ def lut_linear_bwd_x(grad_y, packed, palette, lora_gt=None, lora_a=None, staged=
         rank = lora_gt.shape[1]
         if lora_gt.shape[0] != M or tuple(lora_a.shape) != (rank, K):
             raise ValueError("lora_gt / lora_a shape mismatch")
-    if staged and query("plz_lut_linear_staged", M, K, N) == 1:
-        return linear_bwd_x_dense(grad_y, dequant(packed, palette), lora_gt, lora_a, tiled=True)
     gx = torch.empty((M, K), dtype=torch.bfloat16, device=grad_y.device)
-    q = "plz_lut_linear_bwd_x_workspace" if staged else "plz_linear_bwd_x_dense_workspace"
+    q = "plz_lut_linear_bwd_x_tiled_workspace" if staged else "plz_linear_bwd_x_dense_workspace"
     ws = _opt_workspace(query(q, M, N, K), grad_y.device)
-    call("plz_lut_linear_bwd_x", _ptr(grad_y), _ptr(packed), _ptr(palette), _ptr(lora_gt),
+    call("plz_lut_linear_bwd_x_tiled" if staged else "plz_lut_linear_bwd_x", _ptr(grad_y), _ptr(packed), _ptr(palette), _ptr(lora_gt),
          _ptr(lora_a), rank, _ptr(gx), _ptr(ws), _numel(ws), M, N, K, _stream(grad_y))
     return gx
 

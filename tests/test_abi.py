@@ -281,18 +281,49 @@ def test_forward_mode_tangent_of_the_base_output_is_left_to_the_add():
     (48, 4096, 2560, 0), (128, 4096, 2560, 1), (1000, 4096, 2560, 1), (777, 9728, 2560, 0),
     (4096, 9728, 2560, 2), (128, 9728, 2560, 1), (200, 9728, 2560, 0), (257, 9728, 2560, 1),
     (385, 9728, 2560, 0), (512, 9728, 2560, 0), (640, 9728, 2560, 0), (512, 9728, 1024, 0),
-    (256, 9728, 1024, 1), (2048, 9728, 1024, 1), (640, 9728, 256, 0), (128, 9728, 256, 1),
+    (256, 9728, 1024, 1), (2048, 9728, 1024, 1), (640, 9728, 256, 0),
+    # shorter than the host takes to issue a call
+    (128, 9728, 256, 0), (65, 256, 256, 0), (4095, 264, 512, 0), (100, 1024, 1024, 1),
     (640, 4864, 1280, 1), (640, 3072, 1024, 1), (640, 2560, 9728, 1)])
 def test_lut_gemms_of_wide_outputs_stay_where_they_are_faster(lib, M, J, R, staged):
     if torch.cuda.is_available() and \
             torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("sizes for 256 CUs")
     assert lib.plz_lut_linear_staged(M, J, R) == staged
-    # with grad_x on the same W a wide forward is staged as any other
-    if 128 <= M <= 640:
+    # with grad_x on the same W a wide or short forward is staged as any other
+    if 65 <= M <= 640:
         assert lib.plz_lut_linear_staged_pair(M, J, R) == 1
-    else:
+    elif J * R > 1 << 18:
         assert lib.plz_lut_linear_staged_pair(M, J, R) == staged
+    # the entries that may run so ask for W and the splits' partials, else for what they did
+    w, plain = 2 * J * R, lib.plz_lut_linear_fwd_workspace(M, J, R)
+    got = lib.plz_lut_linear_fwd_tiled_workspace(M, J, R)
+    assert got == (w + lib.plz_linear_tiled_workspace(M, J, R) if staged == 1 else plain)
+    plain = lib.plz_lut_linear_bwd_x_workspace(M, R, J)
+    got = lib.plz_lut_linear_bwd_x_tiled_workspace(M, R, J)
+    assert got == (w + lib.plz_linear_tiled_workspace(M, J, R) if staged == 1 else plain)
+
+
+def test_hard_linears_are_one_call_each_whatever_the_schedule(monkeypatch):
+    """The binding makes one query and one call for a hard forward and for its grad_x at every size:
+    a second call for the dequantised W cost small sizes more than the kernels gained. (CPU tensors as
+    stand-ins: nothing is launched.)"""
+    from palettize_hip import _lib as L, ops
+    calls, queries = [], []
+    monkeypatch.setattr(ops, "_need", lambda t, *a: t)
+    monkeypatch.setattr(ops, "_stream", lambda t: None)
+    monkeypatch.setattr(ops, "call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(ops, "query", lambda name, *a: queries.append(name) or L.query(name, *a))
+    for M, N, K in ((1, 256, 256), (65, 256, 256), (100, 1024, 1024), (777, 512, 2560),
+                    (4096, 256, 2560)):
+        packed = torch.zeros(N, K // 16, dtype=torch.int32)
+        pal, x = torch.zeros(N, K // 256, 4), torch.zeros(M, K, dtype=torch.bfloat16)
+        gy = torch.zeros(M, N, dtype=torch.bfloat16)
+        for staged in (True, False):
+            calls.clear(), queries.clear()
+            ops.lut_linear_fwd(x, packed, pal, staged=staged)
+            ops.lut_linear_bwd_x(gy, packed, pal, staged=staged)
+            assert len(calls) == len(queries) == 2
 
 
 @pytest.mark.parametrize("M,N,K,few_rows", [

@@ -85,9 +85,9 @@ def _oracle_problem(M, N, K, seed, rank=0):
     (4097, 1032, 768, 8),
 ])
 def test_lut_linear_fwd(dev, M, N, K, rank):
-    """The call's own route (from 65 rows here W dequantised and a dense GEMM on it, in the call's
-    workspace from 4096) and the one-pass one."""
-    assert ops.lut_linear_staged(M, N, K) == (M > 64)
+    """The call's own route (from 65 rows and long enough W dequantised into its workspace and a
+    dense GEMM on it) and the one-pass one."""
+    assert ops.lut_linear_staged(M, N, K) == (M > 64 and K > 512)
     idx, pal, x, W, lora = _oracle_problem(M, N, K, seed=M + N + K, rank=rank)
     bias = randn_bf16(N, seed=5, std=0.1) if M % 2 else None
     args = {}
@@ -114,9 +114,9 @@ def test_lut_linear_fwd(dev, M, N, K, rank):
                                         (77, 1032, 768, 8), (256, 384, 1024, 32),
                                         (4096, 1032, 768, 8)])
 def test_lut_linear_bwd_x(dev, M, N, K, rank):
-    """The call's own route (from 65 rows here W dequantised and a dense GEMM on it, in the call's
-    workspace from 4096) and the one-pass one."""
-    assert ops.lut_linear_staged(M, K, N) == (M > 64)
+    """The call's own route (from 65 rows and long enough W dequantised into its workspace and a
+    dense GEMM on it) and the one-pass one."""
+    assert ops.lut_linear_staged(M, K, N) == (M > 64 and N > 512)
     idx, pal, _, W, lora = _oracle_problem(M, N, K, seed=3 * M + N, rank=rank)
     gy = randn_bf16(M, N, seed=9)
     args = {}
