@@ -1739,12 +1739,19 @@ constexpr double kCallUs = 18.5;
 // and dequantise + dense in us, 256 -> 9728 at M = 512 / 640 13.2 / 13.4 and 14.2 / 16.0; 1024 ->
 // 9728 at M = 128 / 256 / 640 28.7 / 28.6 / 28.5 and 28.4 / 24.9 / 34.6; 2560 -> 9728 at M = 128 /
 // 200 / 512 42.3 / 42.3 / 49.1 and 35.5 / 45.2 / 51.7. From 769 rows (2048 of 1024 -> 9728: 64.5 and
-// 56.2) and for 1280 -> 4864 (M = 640: 25.0 and 18.8) the models hold.
+// 56.2) and for 1280 -> 4864 (M = 640: 25.0 and 18.8) the models hold. Square W of more than 2^24
+// weights, too, only while a CU holds one workgroup (5120 -> 5120 at M = 384 / 777 as a forward
+// 55.5 / 71.4 and 48.0 / 74.3, as grad_x 57.4 / 75.8 and 50.1 / 86.1), and one row of tiles is not worth
+// dequantising more than 3 2^24 (9728 x 2560 at 128 rows 38.8 and 35.9; 14336 x 4096 at 65 / 128 rows
+// 50.0 / 52.9 and 56.2 / 56.6).
 static bool staged_alone(int64_t I, int64_t J, int64_t R, int* z = nullptr) {
   if (core256_us(I, J, R, 1.55) < kCallUs || !staged_rows(I, J, R, z)) return false;
-  if (J <= 3 * R || I <= 128 || I > 768) return true;
   const int64_t tiles = ((I + 127) / 128) * ((J + 127) / 128);  // of the 128x128 core
-  return tiles <= cu_count() && (I > 256 || J * R < ((int64_t)1 << 24));
+  const int64_t JR = J * R;
+  if (JR > ((int64_t)1 << 24) && J >= R && (I <= 128 ? JR >= ((int64_t)3 << 24) : tiles > cu_count()))
+    return false;
+  if (J <= 3 * R || I <= 128 || I > 768) return true;
+  return tiles <= cu_count() && (I > 256 || JR < ((int64_t)1 << 24));
 }
 // Tile-rows walked together by the dense GEMMs (consecutive workgroups share an x / grad_y
 // panel within groups of this many tile-rows). Measured on the hard step at M = 16384: 4 (and

@@ -284,17 +284,18 @@ def test_forward_mode_tangent_of_the_base_output_is_left_to_the_add():
     (256, 9728, 1024, 1), (2048, 9728, 1024, 1), (640, 9728, 256, 0),
     # shorter than the host takes to issue a call
     (128, 9728, 256, 0), (65, 256, 256, 0), (4095, 264, 512, 0), (100, 1024, 1024, 1),
+    # large weights that are not narrow: one workgroup per CU, and not too large for one row of tiles
+    (384, 5120, 5120, 1), (777, 5120, 5120, 0), (128, 9728, 2560, 1), (128, 14336, 4096, 0),
+    (65, 13824, 5120, 0), (128, 4096, 14336, 1), (777, 4096, 4096, 1),
     (640, 4864, 1280, 1), (640, 3072, 1024, 1), (640, 2560, 9728, 1)])
 def test_lut_gemms_of_wide_outputs_stay_where_they_are_faster(lib, M, J, R, staged):
     if torch.cuda.is_available() and \
             torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("sizes for 256 CUs")
     assert lib.plz_lut_linear_staged(M, J, R) == staged
-    # with grad_x on the same W a wide or short forward is staged as any other
-    if 65 <= M <= 640:
-        assert lib.plz_lut_linear_staged_pair(M, J, R) == 1
-    elif J * R > 1 << 18:
-        assert lib.plz_lut_linear_staged_pair(M, J, R) == staged
+    # with grad_x on the same W a wide, large or short forward is staged as any other
+    models = 64 < M < 4096 and (M, J) != (777, 9728)
+    assert lib.plz_lut_linear_staged_pair(M, J, R) == (1 if models else staged)
     # the entries that may run so ask for W and the splits' partials, else for what they did
     w, plain = 2 * J * R, lib.plz_lut_linear_fwd_workspace(M, J, R)
     got = lib.plz_lut_linear_fwd_tiled_workspace(M, J, R)
