@@ -1699,9 +1699,20 @@ static int dense_splits(int64_t I, int64_t J, int64_t R, double* us = nullptr) {
   if (us) *us = m ? p.us : big;
   return m ? p.z : 0;
 }
+// Long reductions over W's rows (grad_x: B by columns, in transposing LDS reads) in the first
+// quarter wave of second workgroups of the 128x128 core are faster as split 256x256 tiles, which the
+// model does not see: 128 and 256 core in us, 2048 x 2560 x 4096 61.4 and 58.7, 3500 x 1280 x 4864 65.2
+// and 60.2, 1000 x 5120 x 5120 72.3 and 68.0; 1200 x 4096 x 2560 40.6 and 46.3, 300 x 14336 x 4096 (336
+// workgroups) 60.3 and 68.7, and the same sizes with B by rows 4 to 12% faster on the 128 core.
+static bool cols_on_256(int64_t I, int64_t J, int64_t R) {
+  const int64_t tiles = ((I + 127) / 128) * ((J + 127) / 128), C = cu_count();
+  return R >= 4096 && tiles > C && 4 * tiles <= 5 * C;
+}
 // ... with the workspace at hand: unsplit where it does not hold the splits' partials
-static bool mid_splits(int64_t I, int64_t J, int64_t R, void* workspace, size_t workspace_bytes,
-                       int& z) {
+static bool mid_splits(int64_t I, int64_t J, int64_t R, bool b_col, void* workspace,
+                       size_t workspace_bytes, int& z) {
+  if (b_col && cols_on_256(I, J, R) && workspace && workspace_bytes >= tail_bytes(I, J, R))
+    return false;
   z = dense_splits(I, J, R);
   if (z > 1 && (!workspace || !a16(workspace) || workspace_bytes < mid::workspace(I, J, z))) z = 1;
   return z > 0;
@@ -1709,7 +1720,11 @@ static bool mid_splits(int64_t I, int64_t J, int64_t R, void* workspace, size_t 
 // Workspace of a dense GEMM on the core chosen for its shape.
 static size_t dense_bytes(int64_t I, int64_t J, int64_t R) {
   const int z = dense_splits(I, J, R);
-  return z > 0 ? mid::workspace(I, J, z) : tail_bytes(I, J, R);
+  if (z == 0 || cols_on_256(I, J, R)) {
+    const size_t t = tail_bytes(I, J, R), m = mid::workspace(I, J, z);
+    return t > m ? t : m;
+  }
+  return mid::workspace(I, J, z);
 }
 
 // From this many rows the forward and grad_x dequantise W into the workspace and run the
@@ -1803,9 +1818,10 @@ static bool stage_w(Args& g, const int32_t* packed, const float* palette, int64_
 // and the 128x128 core on it, its partials behind W. One call for both launches: as two calls of
 // the binding small sizes waited for the host (1024 -> 1024 at M = 65 to 256 26.4 to 27.6 us a call,
 // 24.6 in one pass, 19.5 so).
-static size_t lut_mid_bytes(int64_t I, int64_t J, int64_t R, int* splits = nullptr) {
+static size_t lut_mid_bytes(int64_t I, int64_t J, int64_t R, bool b_col, int* splits = nullptr) {
   int z = 0;
-  if (I >= kStagedRows) z = dense_splits(I, J, R);
+  if (b_col && cols_on_256(I, J, R)) z = 0;
+  else if (I >= kStagedRows) z = dense_splits(I, J, R);
   else if (!staged_alone(I, J, R, &z)) z = 0;
   if (splits) *splits = z;
   return z > 0 ? staged_w_bytes(J, R) + mid::workspace(I, J, z) : 0;
@@ -1817,7 +1833,7 @@ static bool lut_mid(mid::Args m, bool b_col, const int32_t* packed, const float*
                     void* stream, int* rc) {
   if (!workspace || !a16(workspace)) return false;
   int z;
-  const size_t need = lut_mid_bytes(m.I, m.J, m.R, &z);
+  const size_t need = lut_mid_bytes(m.I, m.J, m.R, b_col, &z);
   if (need == 0 || workspace_bytes < need) return false;
   uint16_t* w = reinterpret_cast<uint16_t*>(workspace);
   *rc = plz_dequant(packed, palette, w, N, K, stream);
@@ -1954,12 +1970,12 @@ int plz_lut_linear_bwd_x_tiled(const uint16_t* grad_y, const int32_t* packed, co
 }
 
 size_t plz_lut_linear_fwd_tiled_workspace(int64_t M, int64_t N, int64_t K) {
-  const size_t m = M > 0 && N > 0 && K > 0 ? lut_mid_bytes(M, N, K) : 0;
+  const size_t m = M > 0 && N > 0 && K > 0 ? lut_mid_bytes(M, N, K, false) : 0;
   return m > 0 ? m : plz_lut_linear_fwd_workspace(M, N, K);
 }
 
 size_t plz_lut_linear_bwd_x_tiled_workspace(int64_t M, int64_t N, int64_t K) {
-  const size_t m = M > 0 && N > 0 && K > 0 ? lut_mid_bytes(M, K, N) : 0;
+  const size_t m = M > 0 && N > 0 && K > 0 ? lut_mid_bytes(M, K, N, true) : 0;
   return m > 0 ? m : plz_lut_linear_bwd_x_workspace(M, N, K);
 }
 
@@ -2135,7 +2151,7 @@ static int linear_fwd_dense(const uint16_t* x, const uint16_t* w, const uint16_t
   PLZ_REQUIRE(rank == 0 || (lora_t && lora_b && a16(lora_t) && a16(lora_b)),
               "%s: rank > 0 needs 16-byte aligned lora_t and lora_b", what);
   int z;
-  if (tiled && mid_splits(M, N, K, workspace, workspace_bytes, z)) {
+  if (tiled && mid_splits(M, N, K, false, workspace, workspace_bytes, z)) {
     mid::Args m = {x, K, w, K, M, N, K, lora_t, lora_b, rank, y, N, bias, residual, N};
     return mid::launch(m, false, z, cu_count(), workspace, (hipStream_t)stream, what);
   }
@@ -2239,7 +2255,7 @@ static int linear_bwd_x_dense(const uint16_t* grad_y, const uint16_t* w, const u
   PLZ_REQUIRE(rank == 0 || (lora_gt && lora_a && a16(lora_gt) && a16(lora_a)),
               "%s: rank > 0 needs 16-byte aligned lora_gt and lora_a", what);
   int z;
-  if (tiled && mid_splits(M, K, N, workspace, workspace_bytes, z)) {
+  if (tiled && mid_splits(M, K, N, true, workspace, workspace_bytes, z)) {
     mid::Args m = {grad_y, N, w, K, M, K, N, lora_gt, lora_a, rank, grad_x, K, bias,
                    nullptr, 0};
     return mid::launch(m, true, z, cu_count(), workspace, (hipStream_t)stream, what);

@@ -305,6 +305,26 @@ def test_lut_gemms_of_wide_outputs_stay_where_they_are_faster(lib, M, J, R, stag
     assert got == (w + lib.plz_linear_tiled_workspace(M, J, R) if staged == 1 else plain)
 
 
+def test_grad_x_of_long_reductions_just_past_one_wave_is_split_tiles(lib):
+    """128x128 tiles a quarter wave past the CUs with W read by columns over 4096 and more rows: the
+    256x256 core's partials are asked for, and no dequantised W (256 CUs)."""
+    if torch.cuda.is_available() and \
+            torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes for 256 CUs")
+    for M, J, R, cols in ((2048, 2560, 4096, True), (3500, 1280, 4864, True),
+                          (777, 5120, 5120, True), (1200, 4096, 2560, False),
+                          (1500, 4096, 4096, False), (1000, 2560, 4096, False)):
+        tail = lib.plz_linear_bwd_x_dense_workspace(M, R, J)
+        tiled = lib.plz_linear_tiled_workspace(M, J, R)
+        assert (tiled >= tail) if cols else tiled < tail
+        w = lib.plz_lut_linear_bwd_x_tiled_workspace(M, R, J)
+        staged = lib.plz_lut_linear_staged(M, J, R)
+        assert w == (2 * J * R + tiled if staged and not cols else tail)
+        # by rows those are the 128x128 core's, dequantised where that pays
+        w = lib.plz_lut_linear_fwd_tiled_workspace(M, J, R)
+        assert w >= 2 * J * R if staged else w == lib.plz_lut_linear_fwd_workspace(M, J, R)
+
+
 def test_hard_linears_are_one_call_each_whatever_the_schedule(monkeypatch):
     """The binding makes one query and one call for a hard forward and for its grad_x at every size:
     a second call for the dequantised W cost small sizes more than the kernels gained. (CPU tensors as
