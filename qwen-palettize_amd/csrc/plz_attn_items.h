@@ -10,9 +10,9 @@ namespace attn {
 // XCD id % 8, each with its own L2: where the (batch, kv head) pairs divide by 8, each XCD takes
 // an eighth of them and the G query heads of a pair, which walk the same K and V, are neighbours
 // there: with a pair's heads on different XCDs every workgroup fetched its own K and V past the
-// L2s, 0.8 GB in the forward and 1.1 GB in dQ at B32 S512 Hq32 Hkv8 (6 TB/s). Forward 147 -> 141
-// us, dQ 188 -> 179 there; B8 S2048 355 -> 328 and 424 -> 399; one long sequence (B1 S4096) the
-// same. With one query head per kv head every order here keeps a pair on one XCD, and the plain one
+// L2s, 0.8 GB in the forward and 1.1 GB in dQ at B32 S512 Hq32 Hkv8 (6 TB/s), which are 0.30 and
+// 0.57 now. Forward 147 -> 141 us, dQ 188 -> 179 there; B8 S2048 355 -> 328 and 424 -> 399; one
+// long sequence (B1 S4096) the same. With one query head per kv head every order here keeps a pair on one XCD, and the plain one
 // is also the dK/dV kernel's, which finds the pair's Q and dO in that L2: backward at B16 S128
 // 8/8 heads 20.4 us against 21.8, B8 S256 26.2 against 27.8. The dK/dV kernel keeps batch-major
 // pairs: the kv blocks of a pair side by side on an XCD (they walk the same Q and dO) took 211 us

@@ -8,12 +8,12 @@
 //   plz_soft_ref_bwd      dW^T = x^T grad_y [K, N] as fp32 partials from the dW GEMM, then one
 //                         streaming pass that draws the noise again, recomputes P in fp32, writes
 //                         grad_logits (4, K, N) and sums the palette gradient
-// so no plane is transposed and no noise tensor exists: per weight 8 B of logits read and 2 B
-// written forward; 8 B + 4 B per split read and 8 B written backward. Both passes are bound by
+// so no plane is transposed and no noise tensor exists: per weight 8 B of logits read and 2 B (with
+// the logits as read, 10 B) written forward; 8 B + 4 B per split read and 8 B written backward. Both passes are bound by
 // their VALU, half of it quarter-rate (per weight 8 logs, 4 exponentials, 9 32-bit multiplies):
-// 2560 x 4096 in 57 us forward and 72 us backward (105 and 210 MB). A training pass of that linear
-// with LoRA at 2048 rows: 908 us through the native layout (two plane transposes of 206 us, noise
-// drawn into and read from an fp32 tensor) -> 405 us.
+// 2560 x 4096 in 52 us forward, 58 with the copy, and 67 us backward (105, 189 and 210 MB). A training
+// pass of that linear with LoRA at 2048 rows: 920 us through the native layout (two plane
+// transposes of 206 us, noise drawn into and read from an fp32 tensor) -> 350 us.
 #include "plz_soft_ref.h"
 #include "palettize_hip.h"
 

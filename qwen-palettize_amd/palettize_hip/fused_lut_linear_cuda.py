@@ -378,8 +378,8 @@ def _soft_forward(ctx, x, palette, logits, bias, group_size, tau, noise, ste, se
         if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
             # The backward draws P again, so it keeps what the forward read and not the caller's
             # tensors, which an optimizer may write in between: the build writes the logits out
-            # (2560 x 4096: 53.3 -> 54.3 us, where a copy of its own takes 23.7). x, too, is a
-            # copy at the sizes where the native layout pads it.
+            # (2560 x 4096: 50 -> 53 us from the caches, 52 -> 58 from memory; a copy of its own
+            # takes 24). x, too, is a copy at the sizes where the native layout pads it.
             if lg.data_ptr() == logits.data_ptr():
                 copy = torch.empty_like(lg)
             if K % 256 and xc.data_ptr() == x.data_ptr():
