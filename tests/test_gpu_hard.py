@@ -471,3 +471,56 @@ def test_tail_parts_past_the_edge(dev, M, N):
     assert_close(f32(ops.lut_linear_bwd_x(gy.to(dev), p, pl, staged=False)), want,
                  what="grad_x (LUT GEMM)")
     assert_close(f32(ops.linear_bwd_x_dense(gy.to(dev), wd)), want, what="dense grad_x")
+
+
+def test_grad_x_just_past_one_wave_of_small_tiles_runs_the_split_tiles(dev):
+    """270 tiles of 128x128 with W read by columns over 4104 rows (256 CUs): the dense grad_x that may
+    pick its core is the 256x256 core's bit for bit, the LUT one the one-pass GEMM's, and a
+    workspace without room for the split tiles' partials leaves the dense one on the 128x128 core."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes for 256 CUs")
+    M, N, K = 1030, 4104, 3840
+    idx, pal, _, W, (a, b) = _oracle_problem(M, N, K, seed=2, rank=16)
+    gy = randn_bf16(M, N, seed=4)
+    p, pl, g, ad = _packed(idx, dev), pal.to(dev), gy.to(dev), a.to(dev)
+    gt = ops.lora_grad_t(g, b.to(dev), 1.0)
+    w = ops.dequant(p, pl)
+    dense = ops.linear_bwd_x_dense(g, w, gt, ad)
+    assert torch.equal(ops.linear_bwd_x_dense(g, w, gt, ad, tiled=True), dense)
+    lut = ops.lut_linear_bwd_x(g, p, pl, gt, ad, staged=False)
+    assert torch.equal(ops.lut_linear_bwd_x(g, p, pl, gt, ad), lut)
+    small = torch.empty_like(dense)
+    ops.call("plz_linear_bwd_x_tiled", g.data_ptr(), w.data_ptr(), gt.data_ptr(),
+             ad.data_ptr(), 16, small.data_ptr(), None, 0, M, N, K, ops._stream(g))
+    rows = [0, 127, 128, 1023, 1024, 1029]
+    want = O.grad_x(f32(gy[rows]), W) + f32(gt[rows]) @ f32(a)
+    for got, what in ((dense, "256 core"), (lut, "LUT GEMM"), (small, "128 core")):
+        assert_close(f32(got[rows]), want, what=what)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 1032, 768), (65, 256, 256), (128, 1024, 2560)])
+def test_hard_linears_in_a_graph(dev, M, N, K):
+    """Forward and grad_x at staged sizes and a one-pass size, W and the partials in workspaces of the
+    graph's pool: every replay, with other eager work between, is the eager result on new inputs."""
+    idx, pal = make_weight(N, K, seed=N)
+    p, pl = _packed(idx, dev), pal.to(dev)
+    x, gy = (torch.empty(M, n, dtype=torch.bfloat16, device=dev) for n in (K, N))
+
+    def work():
+        return ops.lut_linear_fwd(x, p, pl), ops.lut_linear_bwd_x(gy, p, pl)
+
+    x.zero_(), gy.zero_()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        work()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = work()
+    for i in range(4):
+        x.copy_(randn_bf16(M, K, seed=i)), gy.copy_(randn_bf16(M, N, seed=9 + i))
+        graph.replay()
+        got = [o.clone() for o in outs]
+        for a, b in zip(got, work()):
+            assert torch.equal(a, b)
+        torch.cuda.synchronize()
